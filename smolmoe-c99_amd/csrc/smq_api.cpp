@@ -32,6 +32,7 @@ struct Context {
     float *scalar = nullptr;
     void *argmax_parts = nullptr; /* smq::MAX_ARGMAX_PARTS partials of the two-stage argmax */
     float *scores = nullptr;      /* decode attention scores (heads x context), smq::SCORE_WORKSPACE_BYTES */
+    float *tiles_ws = nullptr;    /* prefill attention scores, smq::TILES_WORKSPACE_BYTES */
     float *mq_ws = nullptr;       /* split-K partial sums of the MFMA prefill GEMM, smq::MQ_WORKSPACE_BYTES */
     hipEvent_t t0 = nullptr, t1 = nullptr;
     int fast = 0;
@@ -263,6 +264,7 @@ smq_status smq_init(int device) {
         return t_status;
     if (!hip_ok(hipMalloc((void **)&g.scores, smq::SCORE_WORKSPACE_BYTES), "hipMalloc")) return t_status;
     if (!hip_ok(hipMalloc((void **)&g.mq_ws, smq::MQ_WORKSPACE_BYTES), "hipMalloc")) return t_status;
+    if (!hip_ok(hipMalloc((void **)&g.tiles_ws, smq::TILES_WORKSPACE_BYTES), "hipMalloc")) return t_status;
     if (!hip_ok(hipEventCreate(&g.t0), "hipEventCreate") || !hip_ok(hipEventCreate(&g.t1), "hipEventCreate"))
         return t_status;
     /* the allocation-free argmax's static partials: their device address, once, with the device current */
@@ -291,6 +293,7 @@ void smq_shutdown(void) {
     (void)hipFree(g.flag);
     (void)hipFree(g.argmax_parts);
     (void)hipFree(g.scores);
+    (void)hipFree(g.tiles_ws);
     (void)hipFree(g.mq_ws);
     (void)hipStreamDestroy(g.own);
     g = Context();
@@ -994,6 +997,30 @@ smq_status smq_rope_kv(float *q, float *k, const float *v, uint32_t ntok, const 
                : t_status;
 }
 
+/* Attention of checked operands. The prefill kernels' score workspace belongs to the library's own stream:
+ * work on another stream, or recorded into a graph (which may be replayed beside eager work), takes the
+ * kernels that need none. One thread at a time enqueues the launches that share it. */
+static smq_status attention_launch(const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
+                                   const smq::AttnShape &sh, uint32_t pos0, const int32_t *pos_dev, float *xd,
+                                   int8_t *xq, const char *who) {
+    static std::mutex mu;
+    std::unique_lock<std::mutex> lock(mu, std::defer_lock);
+    float *ws = nullptr;
+    if (ntok > 1 && g.cur == g.own) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+        if (!hip_ok(hipStreamIsCapturing(g.cur, &capture), who)) return t_status;
+        if (capture == hipStreamCaptureStatusNone) {
+            ws = g.tiles_ws;
+            lock.lock();
+        }
+    }
+    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, g.cur, g.scores, ws,
+                                        ws ? smq::TILES_WORKSPACE_BYTES : 0),
+                  who)
+               ? SMQ_OK
+               : t_status;
+}
+
 smq_status smq_attention(const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
                          const smq_attn_shape *shape, uint32_t pos0, const int32_t *pos_dev) {
     if (!ready()) return t_status;
@@ -1007,11 +1034,7 @@ smq_status smq_attention(const float *q, const float *keys, const float *values,
         !extent_ok(keys, cache, "keys") || !extent_ok(values, cache, "values") ||
         !extent_ok(pos_dev, pos_dev ? 4 : 0, "pos"))
         return t_status;
-    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, nullptr, nullptr, g.cur,
-                                        g.scores),
-                  "attention")
-               ? SMQ_OK
-               : t_status;
+    return attention_launch(q, keys, values, att, ntok, sh, pos0, pos_dev, nullptr, nullptr, "attention");
 }
 
 smq_status smq_attention_q8(const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
@@ -1030,17 +1053,11 @@ smq_status smq_attention_q8(const float *q, const float *keys, const float *valu
         !extent_ok(xq, ntok * nbq * smq::QK, "xq"))
         return t_status;
     if (sh.head_dim % smq::QK == 0) /* each head owns whole blocks: quantized in the same kernel */
-        return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, g.cur,
-                                            g.scores),
-                      "attention_q8")
-                   ? SMQ_OK
-                   : t_status;
-    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, nullptr, nullptr,
-                                        g.cur, g.scores),
-                  "attention_q8") &&
-                   hip_ok(smq::launch_quantize_q8(att, ntok, sh.q_dim, xd, xq, g.flag, g.cur), "attention_q8")
-               ? SMQ_OK
-               : t_status;
+        return attention_launch(q, keys, values, att, ntok, sh, pos0, pos_dev, xd, xq, "attention_q8");
+    if (attention_launch(q, keys, values, att, ntok, sh, pos0, pos_dev, nullptr, nullptr, "attention_q8") != SMQ_OK)
+        return t_status;
+    return hip_ok(smq::launch_quantize_q8(att, ntok, sh.q_dim, xd, xq, g.flag, g.cur), "attention_q8") ? SMQ_OK
+                                                                                                        : t_status;
 }
 
 smq_status smq_attention_rope_q8(float *q, float *k, const float *v, const smq_attn_shape *shape,

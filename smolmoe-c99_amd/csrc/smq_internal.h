@@ -202,7 +202,17 @@ hipError_t launch_rope_kv(float *q, float *k, const float *v, uint32_t ntok, con
 hipError_t launch_attention(const float *q, const float *kcache, const float *vcache, float *att, uint32_t ntok,
                             const AttnShape &sh, uint32_t pos0, const int32_t *pos_dev, int *flag, float *xd,
                             int8_t *xq, hipStream_t s,
-                            float *scores = nullptr);
+                            float *scores = nullptr, float *tiles_ws = nullptr, size_t tiles_ws_bytes = 0);
+/* Prefill attention in 16-row tiles (csrc/smq_attend.hip): scores, softmax and values in three launches per
+ * slab of tokens, the scores in ws. attend_tiles_ok: head sizes that are multiples of 8, 16-byte aligned q
+ * and caches, the workspace holds the score rows of at least one token. */
+constexpr size_t TILES_WORKSPACE_BYTES = (size_t)128 << 20;
+bool attend_tiles_wanted(const AttnShape &sh, uint32_t ntok, uint32_t pos0); /* the rule (smq_kernels.hip) */
+bool attend_tiles_ok(const AttnShape &sh, const float *q, const float *kcache, const float *vcache, uint32_t ntok,
+                     uint32_t pos0, size_t ws_bytes);
+hipError_t launch_attend_tiles(const float *q, const float *kcache, const float *vcache, float *att, uint32_t ntok,
+                               const AttnShape &sh, uint32_t pos0, int *flag, float *xd, int8_t *xq, float *ws,
+                               size_t ws_bytes, hipStream_t s);
 /* One decoding token: RoPE of q and k, the cache store of k and v, and
  * attention (+ Q8 of the row) in one launch; q/k/v are the unrotated QKV
  * outputs. Needs attention_rows_ok (head_dim 64, 16-byte aligned q and

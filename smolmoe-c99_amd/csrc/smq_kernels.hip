@@ -2681,13 +2681,33 @@ bool attention_rows_ok(const AttnShape &sh, const void *q, const void *kcache, c
            ((uintptr_t)vcache & 15) == 0;
 }
 
+/* Whether a prefill's attention is faster in 16-row tiles (three launches, each position's adds of a row in one
+ * wave) than a workgroup per token and KV head or per token, head and 32 columns (one launch, the adds of a
+ * column split from its products). Measured on MI355X, us, tiles / the other:
+ * k_attend_group's shapes by the positions seen: 512 tokens from 0 44.7 / 46.4, 400 from 0 36.3 / 34.4, 512 from
+ * 512 72 / 99, 2 from 1000 36 / 47, 2 from 256 20.2 / 18.2.
+ * The others run about 4 us and 14 (head_dim 128: 26) ns per position in each round of one workgroup per CU,
+ * the tiles 13 us and 25 ns per position while few: 14 heads of 64, 16 tokens from 3800 107 / 112, from 1000
+ * 38 / 33, 64 from 0 16 / 34, 256 from 0 23 / 146; 12 heads of 128, 2 from 3000 87 / 81, 8 from 3000 88 / 156,
+ * 4 from 500 27 / 17, 8 from 500 28 / 33. */
+bool attend_tiles_wanted(const AttnShape &sh, uint32_t ntok, uint32_t pos0) {
+    uint64_t seen = (uint64_t)pos0 + ntok;
+    if (sh.window && sh.window + (uint64_t)ntok < seen) seen = sh.window + (uint64_t)ntok;
+    if (sh.head_dim == AR_HD && sh.context <= AG_MAXP && sh.heads / sh.kv_heads <= AG_MAXG) return seen >= 512;
+    const uint64_t wgs = (uint64_t)ntok * sh.heads * ((sh.head_dim + ATT_JW - 1) / ATT_JW), rounds = (wgs + 255) / 256;
+    return rounds * (4000 + (sh.head_dim <= AR_HD ? 14 : 26) * seen) > 13000 + 25 * seen;
+}
+
 hipError_t launch_attention(const float *q, const float *kcache, const float *vcache, float *att, uint32_t ntok,
                             const AttnShape &sh, uint32_t pos0, const int32_t *pos_dev, int *flag, float *xd,
-                            int8_t *xq, hipStream_t s, float *scores) {
+                            int8_t *xq, hipStream_t s, float *scores, float *tiles_ws, size_t tiles_ws_bytes) {
     if (!ntok) return hipSuccess;
     if (sh.context > MAX_ATT_POSITIONS || sh.head_dim > MAX_HEAD_DIM || sh.head_dim < 1 ||
         (xd && sh.head_dim % QK))
         return hipErrorInvalidValue;
+    if (ntok > 1 && tiles_ws && !pos_dev && g_att_grouped && attend_tiles_wanted(sh, ntok, pos0) &&
+        attend_tiles_ok(sh, q, kcache, vcache, ntok, pos0, tiles_ws_bytes))
+        return launch_attend_tiles(q, kcache, vcache, att, ntok, sh, pos0, flag, xd, xq, tiles_ws, tiles_ws_bytes, s);
     const uint32_t groups = (sh.head_dim + ATT_JW - 1) / ATT_JW;
     if (ntok == 1 && scores && attention_rows_ok(sh, q, kcache, vcache) &&
         (size_t)sh.heads * sh.context <= MAX_SCORE_FLOATS && sh.heads / sh.kv_heads <= AS_MAXG) {
