@@ -11,12 +11,22 @@
  * are packed as 16 nibble bytes (element j low, j + 16 high) after the f16
  * scale and the 32-bit plane of fifth bits (docs/FORMAT.md:124-134).
  *
- * Mapping: half a wave per block. Lane j holds element j (the extreme is a
- * 32-lane reduction over (|x|, -j), so ties keep the first element); lane k < 21
- * then owns candidate k and runs its binary64 error sum over the 32 elements
- * read from LDS in element order, so the 21 serial sums proceed side by side;
- * the winner is the minimum error with ties to the lowest k; lane j quantizes
- * its element with the winner and the half-wave assembles the 22 bytes.
+ * Mapping: a workgroup takes 24 consecutive blocks. Half a wave per block finds the
+ * extreme; then a lane per (block, candidate), 504 of them in two rounds over the 256
+ * threads, runs the binary64 sum over the block's elements in LDS; one lane per block
+ * picks the winner; half a wave per block quantizes and packs into LDS, and the 528
+ * bytes go out as words.
+ *
+ * What bounds it is the 21 x 32 terms per block, so a term is as short as its value
+ * allows. q * d is exact in binary32 (5 and 11 significant bits). x - q * d is exact too:
+ * for q = 0 it is x; otherwise x lies within a factor of two of q * d (Sterbenz). For
+ * |q| >= 2 and the clamped ends that is plain: |x / d| is at most 24.75, even where d is
+ * a subnormal half. For |q| = 1, rint gave 1, so p = fl(x * dinv) is at least 1/2 + 2^-24
+ * and, with both roundings below 2^-24, x / d at least 1/2 (1 - 2^-48): as x and d / 2 are
+ * binary32 numbers, x >= d / 2. The square of a binary32 number is exact in binary64, so
+ * one fused multiply-add is the reference's square, then sum. A term is four binary32
+ * operations, a conversion and that fma. 8960 x 1536: 253.4 us with half a wave per block (21 of 32 lanes) and four
+ * binary64 operations a term -> 71.2 us.
  */
 #include <float.h>
 
@@ -26,8 +36,10 @@
 namespace smq {
 namespace {
 
-constexpr uint32_t CV_WG = 256;                 /* eight blocks per workgroup */
-constexpr uint32_t CV_BLOCKS = CV_WG / 32;
+constexpr uint32_t CV_WG = 256;
+constexpr uint32_t CV_BLOCKS = 24; /* 21 candidates of each: 504 lanes of two rounds */
+constexpr uint32_t CV_K = 21;
+constexpr uint32_t CV_PITCH = 36; /* floats per block: a wave's three or four blocks on distinct banks */
 
 /* lrintf(v * inv) clamped to the 5-bit range (kernels.c:1064-1067). A NaN product takes
  * -16: x86-64's lrintf returns LONG_MIN for it (cvtss2si's "integer indefinite"), which the
@@ -44,88 +56,113 @@ __device__ __forceinline__ uint32_t to_half_bits(float f) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
 }
 
-__global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t rows, uint32_t cols,
-                                                       unsigned char *out) {
-    __shared__ float xs[CV_BLOCKS][32];
-    __shared__ double errs[CV_BLOCKS][32];
-    const uint32_t tid = threadIdx.x, slot = tid / 32, j = tid % 32;
-    const uint32_t nb = (cols + 31) / 32;
-    const uint64_t blk = (uint64_t)blockIdx.x * CV_BLOCKS + slot;
-    const bool live = blk < (uint64_t)rows * nb; /* uniform per half-wave */
-    const uint32_t row = live ? (uint32_t)(blk / nb) : 0, b = live ? (uint32_t)(blk % nb) : 0;
-    const uint32_t n = cols - b * 32 < 32 ? cols - b * 32 : 32; /* elements of this block */
-    const bool valid = live && j < n;
-    const float v = valid ? x[(size_t)row * cols + (size_t)b * 32 + j] : 0.0f;
-    xs[slot][j] = v;
+/* Candidate k's scale as a half (0 or non-finite: skipped). */
+__device__ __forceinline__ uint32_t q5_candidate(float extreme, uint32_t k) {
+    const float t = 0.1f * (float)k;
+    const float divisor = -(14.5f + t);
+    return to_half_bits(extreme / divisor);
+}
 
+__global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t blocks, uint32_t nb, uint32_t cols,
+                                                       unsigned char *out) {
+    __shared__ __attribute__((aligned(16))) float xs[CV_BLOCKS * CV_PITCH];
+    __shared__ double errs[CV_BLOCKS * CV_K];
+    __shared__ float ext[CV_BLOCKS], winv[CV_BLOCKS];
+    __shared__ uint32_t whalf[CV_BLOCKS];
+    __shared__ __attribute__((aligned(4))) unsigned char bytes[CV_BLOCKS * Q5_BYTES];
+    const uint32_t tid = threadIdx.x, j = tid % 32, b0 = blockIdx.x * CV_BLOCKS;
+    constexpr uint32_t U = CV_BLOCKS * 32 / CV_WG;
+    float v[U];
+    bool valid[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t blk = b0 + u * (CV_WG / 32) + tid / 32, row = blk / nb, c = (blk - row * nb) * 32 + j;
+        valid[u] = blk < blocks && c < cols;
+        v[u] = valid[u] ? x[(size_t)row * cols + c] : 0.0f;
+    }
     /* the signed extreme: largest |x|, first on ties (kernels.c:1090-1091); a NaN never wins
      * (fabsf(NaN) > m is false there), so it enters as -1 and an all-NaN block keeps extreme 0 */
-    float best_a = v == v ? fabsf(v) : -1.0f;
-    uint32_t best_j = j;
 #pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) {
-        const float oa = __shfl_xor(best_a, off, 32);
-        const uint32_t oj = __shfl_xor(best_j, off, 32);
-        if (oa > best_a || (oa == best_a && oj < best_j)) {
-            best_a = oa;
-            best_j = oj;
-        }
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t slot = u * (CV_WG / 32) + tid / 32;
+        xs[slot * CV_PITCH + j] = v[u];
+        const float av = v[u] == v[u] ? fabsf(v[u]) : -1.0f, m = max32(av);
+        const uint64_t at = __ballot(av == m);
+        const uint32_t first = (uint32_t)__builtin_ctz((uint32_t)((tid & 63u) < 32 ? at : at >> 32));
+        const float e = __shfl(v[u], (int)first, 32);
+        if (j == 0) ext[slot] = m > 0.0f ? e : 0.0f;
     }
-    __syncthreads(); /* xs */
-    const float extreme = best_a > 0.0f ? xs[slot][best_j] : 0.0f;
+    __syncthreads();
 
-    /* candidate k = lane j < 21: its scale and its error sum in element order (a NaN element
-     * makes every kept candidate's sum NaN) */
-    double err = -1.0; /* skipped: no sum of squares is -1 */
-    float d = 0.0f;
-    uint32_t h = 0;
-    if (extreme != 0.0f && j <= 20) {
-        const float t = 0.1f * (float)j;
-        const float divisor = -(14.5f + t);
-        h = to_half_bits(extreme / divisor);
-        d = half_to_float(h);
-        if (d != 0.0f && fabsf(d) <= FLT_MAX) {
+    /* error sums in element order (a NaN element makes every kept candidate's sum NaN; the zeros past a
+     * short block's end add zeros) */
+    for (uint32_t id = tid; id < CV_BLOCKS * CV_K; id += CV_WG) {
+        const uint32_t slot = id / CV_K, k = id - slot * CV_K;
+        const float extreme = ext[slot];
+        double err = -1.0; /* skipped: no sum of squares is -1 */
+        const float d = half_to_float(q5_candidate(extreme, k));
+        if (extreme != 0.0f && d != 0.0f && fabsf(d) <= FLT_MAX) {
             const float dinv = 1.0f / d;
+            const float4 *x4 = (const float4 *)&xs[slot * CV_PITCH];
             double acc = 0.0;
-            for (uint32_t e = 0; e < n; ++e) { /* uniform trip count; LDS broadcast reads */
-                const float xe = xs[slot][e];
-                const double q = (double)q5_level(xe, dinv);
-                const double pe = q * (double)d;
-                const double de = (double)xe - pe;
-                const double sq = de * de;
-                acc = acc + sq;
+#pragma unroll
+            for (uint32_t g = 0; g < 8; ++g) {
+                const float4 xv = x4[g];
+                const float e4[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const float q = __builtin_amdgcn_fmed3f(__builtin_rintf(e4[i] * dinv), -16.0f, 15.0f);
+                    const double de = (double)__builtin_fmaf(-q, d, e4[i]);
+                    acc = __builtin_fma(de, de, acc);
+                }
             }
             err = acc;
         }
+        errs[id] = err;
     }
-    errs[slot][j] = err;
     __syncthreads();
     /* first minimum over the kept candidates, as `best < 0 || err < best` (kernels.c:1099): the
      * first kept one is taken whatever its error, so NaN sums leave the first kept candidate */
-    uint32_t win = 32;
-    double best = -1.0;
-    for (uint32_t k = 0; k <= 20; ++k) {
-        const double e = errs[slot][k];
-        if (e != -1.0 && (best < 0.0 || e < best)) {
-            best = e;
-            win = k;
+    if (tid < CV_BLOCKS) {
+        uint32_t win = CV_K;
+        double best = -1.0;
+#pragma unroll
+        for (uint32_t k = 0; k < CV_K; ++k) {
+            const double e = errs[tid * CV_K + k];
+            if (e != -1.0 && (best < 0.0 || e < best)) {
+                best = e;
+                win = k;
+            }
         }
+        const uint32_t h = win < CV_K ? q5_candidate(ext[tid], win) : 0u;
+        whalf[tid] = h;
+        winv[tid] = win < CV_K ? 1.0f / half_to_float(h) : 0.0f; /* 0: no scale was kept */
     }
-    const uint32_t wh = __shfl(h, win < 32 ? win : 0, 32);
-    const float wd = win < 32 ? __shfl(d, win, 32) : 0.0f;
-    const uint32_t half = win < 32 ? wh : 0u;
-    const float inv = wd != 0.0f ? 1.0f / wd : 0.0f;
-    const uint32_t u = (uint32_t)((valid && wd != 0.0f ? q5_level(v, inv) : 0) + 16);
+    __syncthreads();
 
     /* pack: high plane bit j = bit 4 of code j; byte 6 + j (j < 16) = code j | code j+16 << 4 */
-    const uint64_t hb = __ballot((u >> 4) & 1u);
-    const uint32_t high = (uint32_t)(((tid & 63u) < 32 ? hb : hb >> 32) & 0xffffffffu);
-    const uint32_t upper = __shfl_down(u, 16, 32);
-    if (!live) return;
-    unsigned char *o = out + (size_t)row * nb * Q5_BYTES + (size_t)b * Q5_BYTES;
-    if (j < 16) o[6 + j] = (unsigned char)((u & 15u) | ((upper & 15u) << 4));
-    else if (j < 18) o[j - 16] = (unsigned char)(half >> (8 * (j - 16)));
-    else if (j < 22) o[2 + (j - 18)] = (unsigned char)(high >> (8 * (j - 18)));
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t slot = u * (CV_WG / 32) + tid / 32;
+        const float inv = winv[slot];
+        const uint32_t q = (uint32_t)((valid[u] && inv != 0.0f ? q5_level(v[u], inv) : 0) + 16);
+        const uint64_t hb = __ballot((q >> 4) & 1u);
+        const uint32_t high = (uint32_t)((tid & 63u) < 32 ? hb : hb >> 32), half = whalf[slot];
+        const uint32_t upper = __shfl_down(q, 16, 32);
+        unsigned char *o = bytes + slot * Q5_BYTES;
+        if (j < 16) o[6 + j] = (unsigned char)((q & 15u) | ((upper & 15u) << 4));
+        else if (j < 18) o[j - 16] = (unsigned char)(half >> (8 * (j - 16)));
+        else if (j < 22) o[2 + (j - 18)] = (unsigned char)(high >> (8 * (j - 18)));
+    }
+    __syncthreads();
+    const uint32_t live = (blocks - b0 < CV_BLOCKS ? blocks - b0 : CV_BLOCKS) * Q5_BYTES;
+    unsigned char *o = out + (size_t)b0 * Q5_BYTES;
+    if (((uintptr_t)out & 3u) == 0) { /* b0 * 22 is a multiple of 528 */
+        if (tid < live / 4) ((uint32_t *)o)[tid] = ((const uint32_t *)bytes)[tid];
+        else if (tid == live / 4 && live % 4) *(uint16_t *)(o + (live & ~3u)) = *(const uint16_t *)(bytes + (live & ~3u));
+    } else {
+        for (uint32_t i = tid; i < live; i += CV_WG) o[i] = bytes[i];
+    }
 }
 
 }  // namespace
@@ -134,8 +171,9 @@ hipError_t launch_quantize_q5(const float *x, uint32_t rows, uint32_t cols, unsi
     const uint64_t blocks = (uint64_t)rows * ((cols + 31) / 32);
     if (!blocks) return hipSuccess;
     const uint64_t grid = (blocks + CV_BLOCKS - 1) / CV_BLOCKS;
-    if (grid > 0x7fffffffu) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_quantize_q5, dim3((uint32_t)grid), dim3(CV_WG), 0, s, x, rows, cols, out);
+    if (blocks > 0xffffffffu - CV_BLOCKS) return hipErrorInvalidValue; /* more than the device memory holds */
+    hipLaunchKernelGGL(k_quantize_q5, dim3((uint32_t)grid), dim3(CV_WG), 0, s, x, (uint32_t)blocks, (cols + 31) / 32, cols,
+                       out);
     return hipGetLastError();
 }
 

@@ -118,3 +118,30 @@ def test_round_trip_bound(orc):
         y = out.download(np.float32)
         scales = np.abs(q[r].reshape(8, 22)[:, :2].copy().view(np.float16).astype(np.float32)).repeat(32)
         assert np.all(np.abs(y - x[r]) <= scales * 1.0001 + 1e-7)
+
+
+@pytest.mark.parametrize("rows,cols,offset", [(1, 1, 0), (25, 31, 0), (7, 33, 0), (3, 1000, 2), (5, 773, 1), (49, 64, 0)])
+def test_block_groups(orc, rows, cols, offset):
+    """24 blocks per workgroup: partial groups, rows that end inside one, short blocks, outputs at any byte."""
+    say("q5 block groups", rows, cols, offset)
+    x = synth.normal(61, rows * cols, 1.0).reshape(rows, cols)
+    n = rows * ((cols + 31) // 32) * 22
+    xb, out = smq.DeviceBuffer.from_array(x), smq.DeviceBuffer(n + offset + 8)
+    out.fill(0xA5)
+    smq.quantize_q5_rows(xb, rows, cols, out.at(offset))
+    got = out.download(np.uint8)
+    assert np.array_equal(got[offset:offset + n].reshape(rows, -1), orc.quantize_q5_rows(x).reshape(rows, -1))
+    assert (got[:offset] == 0xA5).all() and (got[offset + n:] == 0xA5).all()
+
+
+def test_half_steps(orc):
+    """Elements within a few ulps of every half step of the winning scales: where the rounding to a code and the
+    exactness of the error's difference change."""
+    rng = np.random.default_rng(62)
+    x = np.zeros((400, 64), np.float32)
+    for r in range(400):
+        d = np.float32(np.float16(rng.uniform(0.5, 2.0) * 2.0 ** int(rng.integers(-20, 8))))
+        steps = (rng.integers(-33, 34, 64) * np.float32(0.5) * d).astype(np.float32)
+        x[r] = (steps.view(np.int32) + rng.integers(-3, 4, 64)).astype(np.int32).view(np.float32)
+        x[r, ::32] = np.float32(rng.uniform(14.5, 16.5)) * d * (1 if r % 2 else -1)
+    check(orc, x, "half steps")
