@@ -159,26 +159,6 @@ __global__ __launch_bounds__(64 * AP_SW) __attribute__((amdgpu_waves_per_eu(NG <
     }
 }
 
-/* exp_det_tab without a branch (a lane's four run side by side). */
-__device__ __forceinline__ float exp_det_flat(float x, const uint64_t *tab) {
-    const double inv_ln2_n = 0x1.71547652b82fep+5, shift = 0x1.8p+52;
-    const double ea = 0x1.62e42fefa39efp-1 / 32;
-    const double c1 = ea, c2 = ea * ea / 2, c3 = ea * ea * ea / 6, c4 = ea * ea * ea * ea / 24;
-    const float xc = x > 89.0f ? 89.0f : (x < -104.0f ? -104.0f : x);
-    const double z = inv_ln2_n * (double)xc;
-    double kd = z + shift;
-    const uint64_t ki = (uint64_t)__double_as_longlong(kd);
-    kd = kd - shift;
-    const double r = z - kd;
-    double p = c4 * r + c3;
-    p = p * r + c2;
-    p = p * r + c1;
-    p = p * r + 1.0;
-    const double scale = __longlong_as_double((long long)(tab[ki & 31u] + (ki << 47)));
-    const float e = (float)(p * scale);
-    return x != x ? x : e;
-}
-
 /* Softmax weights of one row tile. A wave per row finds the maximum (order-free; NaN never wins). Then 15
  * waves form exp_det(s - max), a group of 16 positions of every row each, written back and to LDS, two
  * chunks of 15 groups requested ahead; the last wave meanwhile adds the previous chunk, a lane per row, in

@@ -480,6 +480,26 @@ __device__ __forceinline__ float exp_det_tab(float x, const uint64_t *tab) {
 
 __device__ __forceinline__ float exp_det(float x) { return exp_det_tab(x, EXP2_TABLE); }
 
+/* exp_det_tab without a branch: several of a thread's run side by side. */
+__device__ __forceinline__ float exp_det_flat(float x, const uint64_t *tab) {
+    const double inv_ln2_n = 0x1.71547652b82fep+5, shift = 0x1.8p+52;
+    const double ea = 0x1.62e42fefa39efp-1 / 32;
+    const double c1 = ea, c2 = ea * ea / 2, c3 = ea * ea * ea / 6, c4 = ea * ea * ea * ea / 24;
+    const float xc = x > 89.0f ? 89.0f : (x < -104.0f ? -104.0f : x);
+    const double z = inv_ln2_n * (double)xc;
+    double kd = z + shift;
+    const uint64_t ki = (uint64_t)__double_as_longlong(kd);
+    kd = kd - shift;
+    const double r = z - kd;
+    double p = c4 * r + c3;
+    p = p * r + c2;
+    p = p * r + c1;
+    p = p * r + 1.0;
+    const double scale = __longlong_as_double((long long)(tab[ki & 31u] + (ki << 47)));
+    const float e = (float)(p * scale);
+    return x != x ? x : e;
+}
+
 /* DPP move of v from another lane of its row of 16 (ctrl: a dpp_ctrl code). */
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {

@@ -984,7 +984,7 @@ __global__ __launch_bounds__(WG) void k_quantize_q8(const float *x, uint32_t row
  * Activation producers (reference: src/model.c:334-415, src/vecmath.c:61-93).
  * One workgroup of NT threads per token row (256 for rows up to 4096
  * elements, so that many rows run at once; 1024 for longer ones; 512 for
- * rows up to 8192 measured no faster on the 4864-wide SwiGLU rows): optional
+ * rows up to 8192 measured no faster on 4864-wide SwiGLU rows): optional
  * RMSNorm (sequential f32 sum of squares, model.c:337 — the squares are formed
  * in parallel, one wave adds them in element order), optional SwiGLU / GeGLU
  * with the binary64 exp below, then the Q8 block quantization of
@@ -1095,6 +1095,68 @@ __global__ __launch_bounds__(NT) void k_row_quantize(const float *src, const flo
             }
         }
     }
+}
+
+/* The same rows without a norm, where they are whole blocks (n % 32 == 0) and so one flat run of
+ * elements: a thread takes four (16-byte reads, one 4-byte write of its int8), eight threads a block, and
+ * every load is issued before the first use. k_row_quantize holds up to sixteen elements of one row per
+ * thread in guarded registers, reads the gate one element at a time and the exp table through the vector
+ * cache. 512 rows of 4864: SwiGLU 10.6 -> 6.4 us (22.7 MB), plain 9.3 -> 3.8; 100 of 11008, GeGLU 13.0 -> 4.2. */
+template <int ACT>
+__global__ __launch_bounds__(WG) void k_rows_flat(const f4v *src, const f4v *gate, uint64_t quads, f4v *yout, float *d,
+                                                  uint32_t *q, int *flag) {
+    __shared__ uint64_t etab[32];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t i = (uint64_t)blockIdx.x * WG + tid;
+    const bool in = i < quads; /* whole blocks of eight threads */
+    const f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f4v v = in ? src[i] : zero, g = zero;
+    if (ACT) {
+        if (in) g = gate[i];
+        if (tid < 32) etab[tid] = EXP2_TABLE[tid];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float gv = g[k];
+            float u = gv;
+            if (ACT == 2) {
+                const float g3 = 0.044715f * gv * gv * gv;
+                u = 1.5957691216f * (gv + g3);
+            }
+            const float den = 1.0f + exp_det_flat(-u, etab);
+            const float sg = gv / den;
+            v[k] = v[k] * sg;
+        }
+    }
+    if (!in) return;
+    if (yout) yout[i] = v;
+    float m = 0.0f;
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float av = fabsf(v[k]);
+        bad |= !(av <= FLT_MAX);
+        m = av > m ? av : m;
+    }
+    float o = dpp_f<0xB1>(m); /* the block's eight threads: lane^1, lane^2, the other quad */
+    m = o > m ? o : m;
+    o = dpp_f<0x4E>(m);
+    m = o > m ? o : m;
+    o = dpp_f<0x141>(m);
+    m = o > m ? o : m;
+    const float scale = m / 127.0f;
+    const float inv = scale >= FLT_MIN ? 1.0f / scale : 0.0f;
+    uint32_t word = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float p = v[k] * inv;
+        int qv = (int)__builtin_rintf(p);
+        qv = qv > 127 ? 127 : (qv < -127 ? -127 : qv);
+        word |= ((uint32_t)qv & 255u) << (8 * k);
+    }
+    q[i] = word;
+    if ((tid & 7u) == 0) d[i / 8] = scale;
+    if (bad && flag) *flag = 1;
 }
 
 /* h[i] = h[i] * (g / (1 + exp_det(-g))) with g = gate[i] (SwiGLU, act 1) or
@@ -2611,11 +2673,26 @@ hipError_t launch_matmul(const MatArgs &a, bool q5, bool fast, hipStream_t s) {
     return fast ? launch_typed<false, true>(a, s) : launch_typed<false, false>(a, s);
 }
 
+/* Rows of whole blocks, 16-byte aligned reads and 4-byte aligned writes: one flat run of elements. */
+static bool rows_flat_ok(const float *src, const float *gate, uint32_t rows, uint32_t n, const float *y, const int8_t *q) {
+    return n % QK == 0 && (((uintptr_t)src | (uintptr_t)gate | (uintptr_t)y) & 15u) == 0 && ((uintptr_t)q & 3u) == 0 &&
+           (uint64_t)rows * n / 4 <= (uint64_t)0x7fffffff * WG;
+}
+template <int ACT>
+static hipError_t launch_rows_flat(const float *src, const float *gate, uint32_t rows, uint32_t n, float *y, float *d,
+                                   int8_t *q, int *flag, hipStream_t s) {
+    const uint64_t quads = (uint64_t)rows * n / 4;
+    hipLaunchKernelGGL(k_rows_flat<ACT>, dim3((uint32_t)((quads + WG - 1) / WG)), dim3(WG), 0, s, (const f4v *)src,
+                       (const f4v *)gate, quads, (f4v *)y, d, (uint32_t *)q, flag);
+    return hipGetLastError();
+}
+
 hipError_t launch_quantize_q8(const float *x, uint32_t rows, uint32_t n, float *d, int8_t *q, int *flag,
                               hipStream_t s) {
     const uint32_t nb = (n + QK - 1) / QK;
     const uint64_t threads = (uint64_t)rows * nb * QK;
     if (!threads) return hipSuccess;
+    if (rows_flat_ok(x, nullptr, rows, n, nullptr, q)) return launch_rows_flat<0>(x, nullptr, rows, n, nullptr, d, q, flag, s);
     hipLaunchKernelGGL(k_quantize_q8, dim3((uint32_t)((threads + WG - 1) / WG)), dim3(WG), 0, s, x, rows, n, nb, d,
                        q, flag);
     return hipGetLastError();
@@ -2625,6 +2702,11 @@ hipError_t launch_row_quantize(const float *src, const float *norm, float eps, c
                                uint32_t rows, uint32_t n, float *y, float *d, int8_t *q, int *flag, hipStream_t s) {
     if (!rows || !n) return hipSuccess;
     if (n > (uint32_t)(RW_WG * RW_EPT)) return hipErrorInvalidValue;
+    if (!norm && rows_flat_ok(src, gate, rows, n, y, q)) {
+        if (act == 1) return launch_rows_flat<1>(src, gate, rows, n, y, d, q, flag, s);
+        if (act == 2) return launch_rows_flat<2>(src, gate, rows, n, y, d, q, flag, s);
+        return launch_rows_flat<0>(src, nullptr, rows, n, y, d, q, flag, s);
+    }
     const size_t lds = norm ? (size_t)((n + 3) & ~3u) * sizeof(float) : 0; /* the squares' whole float4s */
     const dim3 grid(rows);
     const int nt = n <= (uint32_t)(RW_NARROW * RW_EPT) ? RW_NARROW : RW_WG;
