@@ -397,8 +397,6 @@ __device__ __forceinline__ float chain_lds(float s, const float *a, uint32_t n) 
     return chain_lds_strided(s, (const float4 *)a, 1, n);
 }
 
-__device__ __forceinline__ float serial_sum_lds(const float *a, uint32_t n) { return chain_lds(0.0f, a, n); }
-
 /* ((0 + t_0) + t_1) + ... + t_{64K-1} in f32 by one whole wave with every term in registers: lane i
  * holds terms K*i .. K*i+K-1 in t[], and the running sum moves one lane per step (a DPP wave_shr:1
  * operand of the step's first add), so lane i adds its K terms to the sum of lanes 0..i-1. Lane 63
@@ -418,30 +416,57 @@ __device__ __forceinline__ float wave_chain(const float (&t)[K]) {
     }
     return s;
 }
-
-/* ((0 + a[0]) + a[1]) + ... + a[n-1] from LDS (16-byte aligned) by one whole wave through
- * wave_chain: lane i reads its K consecutive terms (K = the smallest of 4, 8, 10, 12, 16 with 64K >= n;
- * -0.0 past n), then the register chain; longer sequences take the LDS chain. Lane 63 ends with the
- * total (every lane of the wave must call, with the same n). */
+/* The same from s0 (a move per step more: lane 0's old value is a register). */
 template <int K>
-__device__ __forceinline__ float wave_chain_lds_k(const float *a, uint32_t n) {
+__device__ __forceinline__ float wave_chain_from(float s0, const float (&t)[K]) {
+    float s = s0;
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+        s = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(s0), __float_as_int(s), 0x138, 0xf, 0xf, false));
+#pragma unroll
+        for (int k = 0; k < K; ++k) s = s + t[k];
+    }
+    return s;
+}
+
+/* Lane i's K consecutive terms of a[0, n) in LDS (16-byte aligned), -0.0 past n. */
+template <int K>
+__device__ __forceinline__ void chain_terms(float (&t)[K], const float *a, uint32_t n) {
     const uint32_t lane = threadIdx.x & 63u;
-    float t[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const uint32_t i = K * lane + k;
         t[k] = i < n ? a[i] : -0.0f;
     }
+}
+template <int K>
+__device__ __forceinline__ float wave_chain_lds_k(const float *a, uint32_t n) {
+    float t[K];
+    chain_terms<K>(t, a, n);
     return wave_chain<K>(t);
 }
+template <int K>
+__device__ __forceinline__ float wave_chain_lds_from(float s0, const float *a, uint32_t n) {
+    float t[K];
+    chain_terms<K>(t, a, n);
+    return wave_chain_from<K>(s0, t);
+}
+/* ((0 + a[0]) + a[1]) + ... + a[n-1] by one whole wave (every lane must call, with the same n), K the smallest of
+ * 4, 8, 10, 12, 16 with 64K >= n; past 1024 terms 1024 at a time, then the rest. Lane 63 ends with the total. (A
+ * chain fed from LDS past 1024 terms: the RMSNorm of one row of 4096 21.2 -> 19.2 us, of 512 rows of 1536
+ * 10.9 -> 9.6.) */
 __device__ __forceinline__ float serial_sum_wave(const float *a, uint32_t n) {
     if (n <= 64 * 4) return wave_chain_lds_k<4>(a, n);
     if (n <= 64 * 8) return wave_chain_lds_k<8>(a, n);
     if (n <= 64 * 10) return wave_chain_lds_k<10>(a, n);
     if (n <= 64 * 12) return wave_chain_lds_k<12>(a, n);
     if (n <= 64 * 16) return wave_chain_lds_k<16>(a, n);
-    const float s = serial_sum_lds(a, n); /* lane-parallel LDS chain: every lane ends with the total */
-    return s;
+    float s = 0.0f;
+    for (; n > 64 * 16; n -= 64 * 16, a += 64 * 16)
+        s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wave_chain_lds_from<16>(s, a, 64 * 16)), 63));
+    if (n <= 64 * 4) return wave_chain_lds_from<4>(s, a, n);
+    if (n <= 64 * 8) return wave_chain_lds_from<8>(s, a, n);
+    return wave_chain_lds_from<16>(s, a, n);
 }
 
 /* 2^(j/32) correctly rounded to binary64, minus j << 47 (vecmath.c:44-52). */
