@@ -48,6 +48,22 @@ thread_local char t_message[1024];
 /* set between smq_capture_begin and smq_capture_end on the capturing thread */
 thread_local bool t_capturing = false;
 
+/* Score workspaces of captured decode attention, each owned by one graph: a graph may be replayed on any stream,
+ * beside eager work and other graphs. ready_ws waits for the open capture (used: it recorded a launch that writes
+ * it); a graph that recorded one takes it along until smq_graph_destroy. */
+struct GraphScores {
+    std::mutex mu;
+    float *ready_ws = nullptr;
+    bool used = false;
+    std::map<void *, float *> of_graph;
+    std::vector<float *> retired; /* of graphs destroyed inside a capture, where nothing may be freed */
+    void release() {              /* not inside a capture; hipFree waits for a replay in flight */
+        for (float *p : retired) (void)hipFree(p);
+        retired.clear();
+    }
+};
+GraphScores g_graph_scores;
+
 /* The library's own allocations (smq_malloc), base -> size: extent checks look here first, so a
  * check needs no runtime call for them, and none at all runs inside a stream capture. */
 std::mutex g_alloc_mu;
@@ -294,6 +310,12 @@ void smq_shutdown(void) {
     (void)hipFree(g.argmax_parts);
     (void)hipFree(g.scores);
     (void)hipFree(g.tiles_ws);
+    {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        g_graph_scores.release();
+        (void)hipFree(g_graph_scores.ready_ws);
+        g_graph_scores.ready_ws = nullptr;
+    }
     (void)hipFree(g.mq_ws);
     (void)hipStreamDestroy(g.own);
     g = Context();
@@ -997,24 +1019,35 @@ smq_status smq_rope_kv(float *q, float *k, const float *v, uint32_t ntok, const 
                : t_status;
 }
 
-/* Attention of checked operands. The prefill kernels' score workspace belongs to the library's own stream:
- * work on another stream, or recorded into a graph (which may be replayed beside eager work), takes the
- * kernels that need none. One thread at a time enqueues the launches that share it. */
+/* Attention of checked operands. The score workspace of the prefill kernels and of decode at head sizes other than
+ * 64 belongs to the library's own stream, or in smq_capture_begin's captures to the graph: work on another stream
+ * or in a capture that the library did not open takes the kernels that need none. One thread at a time enqueues
+ * the launches that share it. */
 static smq_status attention_launch(const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
                                    const smq::AttnShape &sh, uint32_t pos0, const int32_t *pos_dev, float *xd,
                                    int8_t *xq, const char *who) {
     static std::mutex mu;
     std::unique_lock<std::mutex> lock(mu, std::defer_lock);
-    float *ws = nullptr;
-    if (ntok > 1 && g.cur == g.own) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
-        if (!hip_ok(hipStreamIsCapturing(g.cur, &capture), who)) return t_status;
-        if (capture == hipStreamCaptureStatusNone) {
-            ws = g.tiles_ws;
-            lock.lock();
+    float *ws = nullptr, *scores = g.scores;
+    const bool decode_ws = ntok == 1 && smq::attention_decode_split(sh, q, keys, values, pos0, pos_dev);
+    if (decode_ws) scores = nullptr;
+    if ((ntok > 1 || decode_ws) && g.cur == g.own) {
+        if (t_capturing) {
+            if (decode_ws) {
+                std::lock_guard<std::mutex> l(g_graph_scores.mu);
+                scores = g_graph_scores.ready_ws;
+                g_graph_scores.used = scores != nullptr;
+            }
+        } else {
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+            if (!hip_ok(hipStreamIsCapturing(g.cur, &capture), who)) return t_status;
+            if (capture == hipStreamCaptureStatusNone) {
+                (decode_ws ? scores : ws) = g.tiles_ws;
+                lock.lock();
+            }
         }
     }
-    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, g.cur, g.scores, ws,
+    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, g.cur, scores, ws,
                                         ws ? smq::TILES_WORKSPACE_BYTES : 0),
                   who)
                ? SMQ_OK
@@ -1324,6 +1357,17 @@ smq_status smq_memset(void *dst, int value, size_t bytes) {
 smq_status smq_capture_begin(void) {
     if (!ready()) return t_status;
     if (g.cur != g.own) return set_status(SMQ_ERR_STATE, "capture needs the library stream");
+    {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        g_graph_scores.used = false;
+        g_graph_scores.release();
+        /* without it (no memory) the capture records the kernel that needs none */
+        if (!g_graph_scores.ready_ws &&
+            hipMalloc((void **)&g_graph_scores.ready_ws, smq::SCORE_WORKSPACE_BYTES) != hipSuccess) {
+            g_graph_scores.ready_ws = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     /* thread-local mode: a call from this thread that may not be captured (a synchronizing copy, an
      * allocation) fails the capture instead of being recorded or run behind the graph's back */
     if (!hip_ok(hipStreamBeginCapture(g.cur, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
@@ -1340,7 +1384,14 @@ void *smq_capture_end(void) {
     if (!hip_ok(hipStreamEndCapture(g.cur, &graph), "hipStreamEndCapture")) return nullptr;
     const bool ok = hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     (void)hipGraphDestroy(graph);
-    return ok ? (void *)exec : nullptr;
+    if (!ok) return nullptr;
+    std::lock_guard<std::mutex> l(g_graph_scores.mu);
+    if (g_graph_scores.used) {
+        g_graph_scores.of_graph[(void *)exec] = g_graph_scores.ready_ws;
+        g_graph_scores.ready_ws = nullptr;
+        g_graph_scores.used = false;
+    }
+    return (void *)exec;
 }
 
 smq_status smq_graph_launch(void *graph) {
@@ -1350,7 +1401,15 @@ smq_status smq_graph_launch(void *graph) {
 }
 
 void smq_graph_destroy(void *graph) {
-    if (graph) (void)hipGraphExecDestroy((hipGraphExec_t)graph);
+    if (!graph) return;
+    (void)hipGraphExecDestroy((hipGraphExec_t)graph);
+    std::lock_guard<std::mutex> l(g_graph_scores.mu);
+    auto it = g_graph_scores.of_graph.find(graph);
+    if (it != g_graph_scores.of_graph.end()) {
+        g_graph_scores.retired.push_back(it->second);
+        g_graph_scores.of_graph.erase(it);
+    }
+    if (!t_capturing) g_graph_scores.release();
 }
 
 static bool anchor_shape_ok(const void *a, const void *b, size_t bytes, uint32_t wgs, uint32_t threads) {

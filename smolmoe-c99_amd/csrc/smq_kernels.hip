@@ -1595,13 +1595,75 @@ __device__ __forceinline__ void att_load_values(float4 (&pre)[AR_VL], const floa
     }
 }
 
+/* The value columns of more than AR_VP positions: the first wave adds a chunk of AL_VP products per column in
+ * position order while the other seven form the next chunk in the second buffer, the rows of two chunks ahead
+ * requested. (One buffer of AR_VP rows had left products and sums one after the other: 14 heads of 64 at 3001
+ * positions 30.5 -> 25.4 us, at 12001 106 -> 84.) Lane j of the first wave returns column j's sum. */
+constexpr uint32_t AL_VP = 256;                           /* value rows per chunk: whole batches of the chain */
+constexpr uint32_t AL_P = AL_VP + 4;                      /* column pitch, plus 8 floats per four columns (att_col) */
+constexpr uint32_t AL_BUF = ATT_JW * AL_P + ATT_JW / 4 * 8;
+constexpr uint32_t AL_RR = (AR_WG - 64) * 4 / ATT_JW;     /* rows per round of the seven waves */
+constexpr uint32_t AL_VL = (AL_VP + AL_RR - 1) / AL_RR;   /* float4 value loads per thread and chunk */
+static_assert(2 * AL_BUF <= AR_FIXED && AL_P % 32 == 4, "two chunks in the products region, the bank pattern of att_col");
+template <bool ROPE>
+__device__ __forceinline__ float att_long(const float *sc, float *prod, uint32_t np, uint32_t last, float inv,
+                                          const float *vbase, const float *vrope, uint32_t kvd) {
+    const uint32_t tid = threadIdx.x, pt = tid - 64, vrow = pt / (ATT_JW / 4), vcol = (pt % (ATT_JW / 4)) * 4;
+    const bool adds = tid < 64;
+    f4v va[AL_VL], vb[AL_VL];
+    auto load = [&](f4v (&v)[AL_VL], uint32_t p0) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < AL_VL; ++u) {
+            const uint32_t p = p0 + vrow + u * AL_RR, pc = p < np ? p : np - 1;
+            v[u] = *(const f4v *)((ROPE && pc == last) ? vrope + vcol : vbase + (size_t)pc * kvd + vcol);
+        }
+    };
+    auto put = [&](const f4v (&v)[AL_VL], uint32_t p0, uint32_t b) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < AL_VL; ++u) {
+            const uint32_t r = vrow + u * AL_RR, p = p0 + r;
+            if (r < AL_VP && p < np) {
+                const float w = sc[p] * inv;
+                float *c = prod + b * AL_BUF + vcol * AL_P + vcol / 4 * 8 + r;
+                c[0] = w * v[u].x;
+                c[AL_P] = w * v[u].y;
+                c[2 * AL_P] = w * v[u].z;
+                c[3 * AL_P] = w * v[u].w;
+            }
+        }
+    };
+    float o = 0.0f;
+    if (!adds) {
+        load(va, 0);
+        load(vb, AL_VP);
+        put(va, 0, 0);
+        load(va, 2 * AL_VP);
+    }
+    __syncthreads();
+    auto step = [&](uint32_t p0, uint32_t b, f4v (&v)[AL_VL]) __attribute__((always_inline)) {
+        if (adds) { /* whole wave; lanes past the columns repeat them */
+            const uint32_t j = tid % ATT_JW, rows = np - p0 < AL_VP ? np - p0 : AL_VP;
+            o = chain_lds(o, prod + b * AL_BUF + j * AL_P + j / 4 * 8, rows);
+        } else if (p0 + AL_VP < np) {
+            put(v, p0 + AL_VP, b ^ 1u);
+            load(v, p0 + 3 * AL_VP);
+        }
+        __syncthreads();
+    };
+    for (uint32_t p0 = 0; p0 < np; p0 += 2 * AL_VP) {
+        step(p0, 0, vb);
+        if (p0 + AL_VP < np) step(p0 + AL_VP, 1, va);
+    }
+    return o;
+}
+
 /* Steps 2-4 of the row attention once the scaled scores sc[0, np) are in LDS
  * and each thread holds the maximum of its own (high): the maximum
  * (order-free, NaN never wins as in softmax_inv, kernels.c:1146-1148),
  * exp_det(s - max) in parallel, the total in position order by one lane,
- * then the products (s_p*inv)*v_p[j] of AR_VP rows at a time to LDS and lane
- * j's sum of its column in position order (kernels.c:1165), the next rows
- * loading meanwhile. pre holds the first value rows. The 32 outputs go to
+ * then the products (s_p*inv)*v_p[j] to LDS and lane j's sum of its column in
+ * position order (kernels.c:1165); past AR_VP positions by att_long. pre holds
+ * the value rows (up to AR_VP positions). The 32 outputs go to
  * out[0, 32); with xd, their Q8 block to *xd / xq[0, 32) (kernels.c:912-935). */
 template <bool ROPE>
 __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uint32_t np, uint32_t last,
@@ -1630,12 +1692,14 @@ __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uin
     const float inv = *s_inv;
 
     float o = 0.0f;
-    for (uint32_t p0 = 0; p0 < np; p0 += AR_VP) {
+    if (np > AR_VP) { /* uniform */
+        o = att_long<ROPE>(sc, prod, np, last, inv, vbase, vrope, kvd);
+    } else {
 #pragma unroll
         for (uint32_t u = 0; u < AR_VL; ++u) { /* kernels.c:1165: w = scores[p] * inv, then w * v[j] */
-            const uint32_t r = vrow + u * (AR_WG * 4 / ATT_JW), p = p0 + r;
-            if (p < np) {
-                const float w = sc[p] * inv;
+            const uint32_t r = vrow + u * (AR_WG * 4 / ATT_JW);
+            if (r < np) {
+                const float w = sc[r] * inv;
                 prod[att_col(vcol + 0) + r] = w * pre[u].x;
                 prod[att_col(vcol + 1) + r] = w * pre[u].y;
                 prod[att_col(vcol + 2) + r] = w * pre[u].z;
@@ -1643,15 +1707,7 @@ __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uin
             }
         }
         __syncthreads();
-        if (p0 + AR_VP < np) /* next pass in flight during the sums */
-            att_load_values<ROPE>(pre, vbase, vrope, kvd, p0 + AR_VP, np, last, vrow, vcol);
-        if (tid < ATT_JW) {
-            const uint32_t rows = np - p0 < AR_VP ? np - p0 : AR_VP;
-            const float *colp = prod + att_col(tid);
-            float acc = o;
-            acc = chain_lds(acc, colp, rows); /* kernels.c:1165, position order */
-            o = acc;
-        }
+        if (tid < ATT_JW) o = chain_lds(o, prod + att_col(tid), np); /* kernels.c:1165, position order */
         __syncthreads();
     }
     if (tid < ATT_JW) {
@@ -1727,7 +1783,7 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
     f4v kr[AR_KU];
     att_rows_keys(kr, kbase, kvd, 0, np, ROPE ? last : np, krow, kcol);
     const float *vrope = ROPE ? rr.v + (size_t)kh * AR_HD + j0 : nullptr;
-    att_load_values<ROPE>(pre, vbase, vrope, kvd, 0, np, last, vrow, vcol);
+    if (np <= AR_VP) att_load_values<ROPE>(pre, vbase, vrope, kvd, 0, np, last, vrow, vcol); /* uniform */
     if (rload) rtab[rhalf * (AR_HD / 2) + rj] = rv;
     if (ROPE) __syncthreads(); /* the table rows, before q and k are rotated */
     if (kown) {
@@ -1891,9 +1947,57 @@ __global__ __launch_bounds__(AS_WG) void k_attend_scores(const float *q, float *
     }
 }
 
+/* The scores of other head sizes (multiples of 8): the same pairs of threads, the head's size at run time. */
+__global__ __launch_bounds__(AS_WG) void k_attend_scores_hd(const float *q, const float *kcache, AttnShape sh,
+                                                            uint32_t pos0, const int32_t *pos_dev, int *flag,
+                                                            float *scores) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const uint32_t tid = threadIdx.x, grp = sh.heads / sh.kv_heads, kh = blockIdx.y, kvd = sh.kv_dim, hd = sh.head_dim;
+    const uint32_t pos = pos_dev ? (uint32_t)*pos_dev : pos0;
+    if (pos >= sh.context) {
+        if (tid == 0 && blockIdx.x == 0 && flag) *flag = 1;
+        return;
+    }
+    const uint32_t start = sh.window && pos >= sh.window ? pos - sh.window + 1 : 0, np = pos - start + 1;
+    const uint32_t p0 = blockIdx.x * AS_SP;
+    if (p0 >= np) return; /* uniform: past the current position */
+    const uint32_t cnt = np - p0 < AS_SP ? np - p0 : AS_SP, q4n = hd / 4, pitch = hd + 4;
+    float *kt = lds, *qs = lds + AS_SP * pitch; /* pitch: an odd number of 16-byte pieces */
+    const float *kbase = kcache + (size_t)(start + p0) * kvd + (size_t)kh * hd, *qg = q + (size_t)kh * grp * hd;
+    for (uint32_t f = tid; f < cnt * q4n; f += AS_WG) {
+        const uint32_t r = f / q4n, c = f - r * q4n;
+        *(f4v *)&kt[r * pitch + 4 * c] = *(const f4v *)(kbase + (size_t)r * kvd + 4 * c);
+    }
+    for (uint32_t f = tid; f < grp * q4n; f += AS_WG) *(f4v *)&qs[4 * f] = *(const f4v *)(qg + 4 * f);
+    __syncthreads();
+    const float factor = 1.0f / sqrtf((float)hd);
+    for (uint32_t i = tid; i < 2 * cnt * grp; i += AS_WG) { /* pairs of lanes stay together */
+        const uint32_t d = i / 2, half = i & 1u, hh = d / cnt, r = d - hh * cnt;
+        const f4v *kr = (const f4v *)&kt[r * pitch], *q4 = (const f4v *)&qs[hh * hd];
+        float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+#pragma unroll 4
+        for (uint32_t e = 0; e < hd / 8; ++e) {
+            const f4v kv = kr[2 * e + half], qv = q4[2 * e + half];
+            float p;
+            p = qv.x * kv.x; a0 = a0 + p;
+            p = qv.y * kv.y; a1 = a1 + p;
+            p = qv.z * kv.z; a2 = a2 + p;
+            p = qv.w * kv.w; a3 = a3 + p;
+        }
+        const float b0 = __shfl_xor(a0, 1, 64), b1 = __shfl_xor(a1, 1, 64), b2 = __shfl_xor(a2, 1, 64),
+                    b3 = __shfl_xor(a3, 1, 64);
+        if (!half) {
+            const float p04 = a0 + b0, p15 = a1 + b1, p26 = a2 + b2, p37 = a3 + b3;
+            const float e2 = p04 + p26, o2 = p15 + p37;
+            scores[(size_t)(kh * grp + hh) * sh.context + p0 + r] = (e2 + o2) * factor;
+        }
+    }
+}
+
 /* k_attend_values: workgroup (head, 32 coordinates) loads its scores row and
- * its value rows up front, then steps 2-4 of the row attention (att_tail). */
-template <bool ROPE>
+ * its value rows up front, then steps 2-4 of the row attention (att_tail). HD: the
+ * head size, or 0 for a multiple of 32 read at run time. */
+template <bool ROPE, uint32_t HD>
 __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_attend_values(
     const float *vcache, float *att, AttnShape sh, uint32_t pos0, const int32_t *pos_dev, float *xd, int8_t *xq,
     const float *vraw, const float *scores, int *flag) {
@@ -1901,7 +2005,7 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
     __shared__ uint64_t etab[32];
     __shared__ float red[AR_WG / 64];
     __shared__ float s_inv;
-    constexpr uint32_t ngrp = AR_HD / ATT_JW;
+    const uint32_t hd = HD ? HD : sh.head_dim, ngrp = hd / ATT_JW;
     const uint32_t tid = threadIdx.x, g = blockIdx.x % ngrp, h = blockIdx.x / ngrp;
     const uint32_t kh = h / (sh.heads / sh.kv_heads), kvd = sh.kv_dim, j0 = g * ATT_JW;
     const uint32_t pos = pos_dev ? (uint32_t)*pos_dev : pos0;
@@ -1910,8 +2014,8 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
     const uint32_t last = np - 1;
     float *sc = lds;
     float *prod = lds + ((sh.context + 3) & ~3u);
-    const float *vbase = vcache + (size_t)start * kvd + (size_t)kh * AR_HD + j0;
-    const float *vrope = ROPE ? vraw + (size_t)kh * AR_HD + j0 : nullptr;
+    const float *vbase = vcache + (size_t)start * kvd + (size_t)kh * hd + j0;
+    const float *vrope = ROPE ? vraw + (size_t)kh * hd + j0 : nullptr;
     const float *srow = scores + (size_t)h * sh.context;
     const uint32_t vrow = tid / (ATT_JW / 4), vcol = (tid % (ATT_JW / 4)) * 4;
 
@@ -1926,7 +2030,7 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
         sv[u] = p < np ? srow[p] : 0.0f;
     }
     float4 pre[AR_VL];
-    att_load_values<ROPE>(pre, vbase, vrope, kvd, 0, np, last, vrow, vcol);
+    if (np <= AR_VP) att_load_values<ROPE>(pre, vbase, vrope, kvd, 0, np, last, vrow, vcol); /* uniform */
     if (tid < 32) etab[tid] = ev;
     float high = -FLT_MAX;
 #pragma unroll
@@ -1942,9 +2046,9 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
         sc[p] = v;
         high = v > high ? v : high;
     }
-    const uint32_t blk = (h * AR_HD + j0) / QK;
+    const uint32_t blk = (h * hd + j0) / QK;
     att_tail<ROPE>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, &s_inv,
-                   att + (size_t)h * AR_HD + j0, xd ? xd + blk : nullptr, xq ? xq + (size_t)blk * QK : nullptr, flag);
+                   att + (size_t)h * hd + j0, xd ? xd + blk : nullptr, xq ? xq + (size_t)blk * QK : nullptr, flag);
 }
 
 /* Prefill attention (many tokens, head_dim 64): workgroup (token, KV head)
@@ -2763,6 +2867,21 @@ bool attention_rows_ok(const AttnShape &sh, const void *q, const void *kcache, c
            ((uintptr_t)vcache & 15) == 0;
 }
 
+/* One token at head sizes other than 64 in two launches, from the position where they beat k_attend's one workgroup
+ * per head and 32 columns. Measured on MI355X, us, two launches / one: 12 heads of 128 at 41 positions 8.7 / 7.1, 101
+ * 8.8 / 8.3, 201 8.8 / 10.3, 401 10.4 / 14.9, 3072 26 / 83; 9 heads of 32 at 201 8.6 / 7.9, 301 9.1 / 10.3; 4 heads
+ * of 256 at 41 8.9 / 8.8; 32 heads of 128 at 501 10.9 / 19. A position in device memory counts as past the line:
+ * the context tells what it may reach. */
+bool attention_decode_split(const AttnShape &sh, const void *q, const void *kcache, const void *vcache, uint32_t pos0,
+                            bool pos_dev) {
+    static_assert((AS_SP * (MAX_HEAD_DIM + 4) + AS_MAXG * MAX_HEAD_DIM) * sizeof(float) <= 64 * 1024, "k_attend_scores_hd's LDS");
+    uint32_t seen = pos_dev ? sh.context : pos0 + 1;
+    if (sh.window && seen > sh.window) seen = sh.window;
+    return sh.head_dim != AR_HD && sh.head_dim % ATT_JW == 0 && seen + sh.head_dim >= 280 &&
+           (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) & 15u) == 0 &&
+           (size_t)sh.heads * sh.context <= MAX_SCORE_FLOATS && sh.heads / sh.kv_heads <= AS_MAXG;
+}
+
 /* Whether a prefill's attention is faster in 16-row tiles (three launches, each position's adds of a row in one
  * wave) than a workgroup per token and KV head or per token, head and 32 columns (one launch, the adds of a
  * column split from its products). Measured on MI355X, us, tiles / the other:
@@ -2800,7 +2919,17 @@ hipError_t launch_attention(const float *q, const float *kcache, const float *vc
         const dim3 sgrid((sh.context + AS_SP - 1) / AS_SP, sh.kv_heads);
         hipLaunchKernelGGL(k_attend_scores<false>, sgrid, dim3(AS_WG), 0, s, q, (float *)kcache, (float *)vcache, sh,
                            pos0, pos_dev, flag, none, scores);
-        hipLaunchKernelGGL(k_attend_values<false>, dim3(sh.heads * groups), dim3(AR_WG), lds, s, vcache, att, sh, pos0,
+        hipLaunchKernelGGL((k_attend_values<false, AR_HD>), dim3(sh.heads * groups), dim3(AR_WG), lds, s, vcache, att, sh, pos0,
+                           pos_dev, xd, xq, nullptr, scores, flag);
+        return hipGetLastError();
+    }
+    if (ntok == 1 && scores && attention_decode_split(sh, q, kcache, vcache, pos0, pos_dev)) {
+        /* the same two launches at another head size */
+        const size_t lds = (((size_t)sh.context + 3) / 4 * 4 + (size_t)AR_FIXED) * sizeof(float);
+        const size_t slds = (AS_SP * (size_t)(sh.head_dim + 4) + (size_t)sh.heads / sh.kv_heads * sh.head_dim) * sizeof(float);
+        hipLaunchKernelGGL(k_attend_scores_hd, dim3((sh.context + AS_SP - 1) / AS_SP, sh.kv_heads), dim3(AS_WG), slds, s, q,
+                           kcache, sh, pos0, pos_dev, flag, scores);
+        hipLaunchKernelGGL((k_attend_values<false, 0>), dim3(sh.heads * groups), dim3(AR_WG), lds, s, vcache, att, sh, pos0,
                            pos_dev, xd, xq, nullptr, scores, flag);
         return hipGetLastError();
     }
@@ -2832,8 +2961,9 @@ hipError_t prepare_attention_attributes() {
     const hipError_t es[] = {
         hipFuncSetAttribute((const void *)k_attend_rows<false>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
         hipFuncSetAttribute((const void *)k_attend_rows<true>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
-        hipFuncSetAttribute((const void *)k_attend_values<true>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
-        hipFuncSetAttribute((const void *)k_attend_values<false>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
+        hipFuncSetAttribute((const void *)k_attend_values<true, AR_HD>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
+        hipFuncSetAttribute((const void *)k_attend_values<false, AR_HD>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
+        hipFuncSetAttribute((const void *)k_attend_values<false, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
         hipFuncSetAttribute((const void *)k_attend, hipFuncAttributeMaxDynamicSharedMemorySize, tiled)};
     for (hipError_t e : es)
         if (e != hipSuccess) return e;
@@ -2854,7 +2984,7 @@ hipError_t launch_attention_rope(const float *q, const float *k, const float *v,
         const dim3 sgrid((sh.context + AS_SP - 1) / AS_SP, sh.kv_heads);
         hipLaunchKernelGGL(k_attend_scores<true>, sgrid, dim3(AS_WG), 0, s, q, kcache, vcache, sh, pos0, pos_dev, flag,
                            rr, scores);
-        hipLaunchKernelGGL(k_attend_values<true>, dim3(sh.heads * groups), dim3(AR_WG), lds, s, vcache, att, sh, pos0,
+        hipLaunchKernelGGL((k_attend_values<true, AR_HD>), dim3(sh.heads * groups), dim3(AR_WG), lds, s, vcache, att, sh, pos0,
                            pos_dev, xd, xq, v, scores, flag);
         return hipGetLastError();
     }
