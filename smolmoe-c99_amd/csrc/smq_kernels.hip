@@ -152,6 +152,126 @@ __global__ __launch_bounds__(WG) void k_gemv(MatArgs a) {
 }
 
 /* ------------------------------------------------------------------------
+ * 2-16 tokens against few or long rows, FEW_NT tokens per pass: k_gemv's tasks, each with its block's words of every
+ * token of the pass. The products spread over all threads and only the adds stay serial, a thread per (token, row,
+ * lane), where a thread per output (k_gemm_exact) leaves few rows a serial chain of products and a chunk of 16 blocks
+ * in flight: 896x4864 at 4 tokens 22.5 -> 6.3 us, Q5 1536x8960 at 4 39.3 -> 10.5, 2048x2048 at 8 11.9 -> 6.2. A task
+ * decodes its weights once for all passes; the next pass's or chunk's loads are in flight during the products and
+ * adds. What bounds it with many rows is the LDS traffic of the products, a write and a read each: few_wanted.
+ * ---------------------------------------------------------------------- */
+constexpr int FEW_NT = 4; /* tokens per pass */
+template <bool Q5, bool FAST, int RT, int NG>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_gemv_few(MatArgs a) {
+    constexpr int TB = Q5 ? 2 : 1, TPR = WG / RT, CB = TPR * TB, GS = RT * 32 + 4, NW = Q5 ? 11 : 9, NX = TB * 2;
+    constexpr int CHAINS = RT * 8 * FEW_NT;
+    static_assert(CHAINS <= WG, "a thread per (token, row, lane)");
+    constexpr int DS = RT * 4 + 4;  /* fast mode: scales per group */
+    constexpr int PT = CB / 4 * GS; /* floats of one token's products */
+    constexpr int DT = CB / 4 * DS; /* and of its scales */
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+
+    const uint32_t nb = a.nb, tid = threadIdx.x;
+    const Item I = pick_item(a, blockIdx.x);
+    const uint32_t r0 = (blockIdx.x - I.tile_begin) * RT;
+    const uint32_t tr = tid / TPR, ti = tid % TPR;
+    const bool row_ok = r0 + tr < I.rows;
+    const unsigned char *wrow = I.w + (size_t)(row_ok ? r0 + tr : 0) * I.row_bytes;
+    const uint32_t nchunks = (nb + CB - 1) / CB;
+
+    uint32_t wr[NW];
+    u4a xr[FEW_NT][NX];
+    float xs[FEW_NT][TB];
+    auto load_w = [&](uint32_t b) __attribute__((always_inline)) { /* past the row: its first blocks, not used */
+        const unsigned char *p = wrow + (size_t)(b < nb ? b : 0) * (Q5 ? Q5_BYTES : Q8_BYTES);
+        const u4a v0 = *(const u4a *)p, v1 = *(const u4a *)(p + 16);
+        wr[0] = v0.x; wr[1] = v0.y; wr[2] = v0.z; wr[3] = v0.w;
+        wr[4] = v1.x; wr[5] = v1.y; wr[6] = v1.z; wr[7] = v1.w;
+        if constexpr (Q5) {
+            const u3a v2 = *(const u3a *)(p + 32);
+            wr[8] = v2.x; wr[9] = v2.y; wr[10] = v2.z;
+        } else {
+            wr[8] = *(const uint32_t *)(p + 32);
+        }
+    };
+    auto load_x = [&](uint32_t b, uint32_t g) __attribute__((always_inline)) { /* past the batch: its last token */
+        const uint32_t bc = b < nb ? b : 0;
+#pragma unroll
+        for (int t = 0; t < FEW_NT; ++t) {
+            const uint32_t tok = g * FEW_NT + t < a.ntok ? g * FEW_NT + t : a.ntok - 1;
+            const size_t xb = (size_t)tok * a.xstride + bc;
+#pragma unroll
+            for (int k = 0; k < NX; ++k) xr[t][k] = *(const u4a *)(a.xq + xb * QK + 16 * k);
+#pragma unroll
+            for (int k = 0; k < TB; ++k) xs[t][k] = a.xd[xb + k];
+        }
+    };
+    load_w(ti * TB);
+    load_x(ti * TB, 0);
+
+    const uint32_t ct = tid / (RT * 8), cr = tid % (RT * 8); /* the chain's token of the pass, its row and lane */
+    float acc[NG] = {};
+    uint32_t words[TB][8];
+    float wsc[TB];
+    for (uint32_t c = 0; c < nchunks; ++c) {
+        const uint32_t bt = c * CB + ti * TB;
+        Q5Fields f[2];
+        if (Q5) q5_parse_pair(wr, f[0], f[1]);
+#pragma unroll
+        for (int k = 0; k < TB; ++k) {
+            wsc[k] = Q5 ? f[k].scale : __uint_as_float(wr[0]);
+#pragma unroll
+            for (int l = 0; l < 8; ++l) words[k][l] = Q5 ? q5_signed(f[k], l) : wr[1 + l];
+        }
+        if (c + 1 < nchunks) load_w(bt + CB);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (g && (uint32_t)g * FEW_NT >= a.ntok) break; /* uniform */
+            const bool more = g + 1 < NG && (uint32_t)(g + 1) * FEW_NT < a.ntok;
+            if (row_ok && bt < nb) {
+#pragma unroll
+                for (int t = 0; t < FEW_NT; ++t) {
+#pragma unroll
+                    for (int k = 0; k < TB; ++k) {
+                        const uint32_t bb = ti * TB + k;
+                        const u4a x0 = xr[t][2 * k], x1 = xr[t][2 * k + 1];
+                        const uint32_t x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                        const float d = wsc[k] * xs[t][k];
+                        float *dst = lds + t * PT + (bb / 4) * GS + tr * 32 + (bb % 4);
+#pragma unroll
+                        for (int l = 0; l < 8; ++l) {
+                            const float f = (float)dot4(words[k][l], x[l], 0);
+                            dst[l * 4] = FAST ? f : d * f;
+                        }
+                        if (FAST) lds[FEW_NT * PT + t * DT + (bb / 4) * DS + tr * 4 + (bb % 4)] = d;
+                    }
+                }
+            }
+            if (more) load_x(bt, g + 1);
+            else if (c + 1 < nchunks) load_x(bt + CB, 0);
+            __syncthreads();
+            if (tid < CHAINS) {
+                const uint32_t count = nb - c * CB < (uint32_t)CB ? nb - c * CB : (uint32_t)CB;
+                const float4 *pp = (const float4 *)(lds + ct * PT) + cr;
+                const float4 *dp = FAST ? (const float4 *)(lds + FEW_NT * PT + ct * DT) + cr / 8 : nullptr;
+                if (CB <= 32 && count % 4 == 0)
+                    chain_sum_padded<FAST, CB / 4 <= 8 ? CB / 4 : 8>(acc[g], pp, GS / 4, dp, DS / 4, count / 4);
+                else
+                    chain_sum<FAST, CB / 4>(acc[g], pp, GS / 4, dp, DS / 4, count);
+            }
+            if (more || c + 1 < nchunks) __syncthreads();
+        }
+    }
+    if (tid < CHAINS) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const float v = reduce8_to_lane7(acc[g]);
+            const uint32_t r = r0 + cr / 8, t = g * FEW_NT + ct;
+            if ((tid & 7) == 7 && r < I.rows && t < a.ntok) store_out(I, a.flag, t, r, v);
+        }
+    }
+}
+
+/* ------------------------------------------------------------------------
  * Pinned streaming GEMV (Q8 nb <= MAX_FAST_NB; Q5 nb even, <= MAX_FAST_NB):
  * each workgroup belongs to one item (the launcher gives every item a share
  * of the resident workgroups in proportion to its rows) and walks a
@@ -2454,6 +2574,62 @@ hipError_t launch_gemv_tile(MatArgs a, int rt, hipStream_t s) {
     }
 }
 
+template <bool Q5, bool FAST, int RT>
+constexpr size_t few_lds() {
+    return sizeof(float) * FEW_NT * (WG / RT * (Q5 ? 2 : 1) / 4) * (RT * 32 + 4 + (FAST ? RT * 4 + 4 : 0));
+}
+template <bool Q5, bool FAST, int RT>
+hipError_t prepare_few_rt() {
+    const void *k[] = {(const void *)k_gemv_few<Q5, FAST, RT, 1>, (const void *)k_gemv_few<Q5, FAST, RT, 2>,
+                       (const void *)k_gemv_few<Q5, FAST, RT, 4>};
+    for (const void *f : k) {
+        const hipError_t e =
+            hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)few_lds<Q5, FAST, RT>());
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+template <bool Q5, bool FAST>
+hipError_t prepare_few() {
+    const hipError_t e = prepare_few_rt<Q5, FAST, 4>();
+    return e != hipSuccess ? e : prepare_few_rt<Q5, FAST, 8>();
+}
+template <bool Q5, bool FAST, int RT>
+hipError_t launch_few_rt(MatArgs a, hipStream_t s) {
+    uint32_t tiles = 0;
+    for (uint32_t i = 0; i < a.nitems; ++i) {
+        a.item[i].tile_begin = tiles;
+        tiles += (a.item[i].rows + RT - 1) / RT;
+    }
+    constexpr size_t lds = few_lds<Q5, FAST, RT>();
+    if (a.ntok <= FEW_NT) hipLaunchKernelGGL((k_gemv_few<Q5, FAST, RT, 1>), dim3(tiles), dim3(WG), lds, s, a);
+    else if (a.ntok <= 2 * FEW_NT) hipLaunchKernelGGL((k_gemv_few<Q5, FAST, RT, 2>), dim3(tiles), dim3(WG), lds, s, a);
+    else hipLaunchKernelGGL((k_gemv_few<Q5, FAST, RT, 4>), dim3(tiles), dim3(WG), lds, s, a);
+    return hipGetLastError();
+}
+/* Eight rows per workgroup while one chunk covers the row, else four (more workgroups, longer chunks), except Q5 from
+ * 2048 rows on. Measured (us, four / eight rows): Q5 512x8960 at 4 tokens 8.7 / 12.3, 2048x8960 12.1 / 13.0, 4096x8960
+ * 20.7 / 17.9; Q8 512x4864 6.3 / 8.9, 4096x4864 10.0 / 11.1; 16384x896 11.9 / 9.6; Q5 8960x1536 15.7 / 10.8. */
+template <bool Q5, bool FAST>
+hipError_t launch_few(MatArgs a, uint32_t total_rows, hipStream_t s) {
+    if (a.nb <= (Q5 ? 64u : 32u) || (Q5 && total_rows > 2048)) return launch_few_rt<Q5, FAST, 8>(a, s);
+    return launch_few_rt<Q5, FAST, 4>(a, s);
+}
+/* Where k_gemv_few beats the tiles of k_gemm_exact and k_gemm_xm, by its passes of four tokens: a row of about 16
+ * blocks per pass, and rows x passes up to 8192 (Q5 rows under 48 blocks, which leave tasks of its one chunk idle,
+ * 4096); one pass up to 16384 rows (Q5 12288). Measured on MI355X (us, k_gemv_few / the best tile kernel): one pass:
+ * 16384x896 9.4 / 9.7, 24576x896 12.4 / 11.9, 16384x3072 18.6 / 23.0, 32768x3072 38.4 / 37.2, Q5 8192x896 8.7 / 6.8,
+ * 4096x896 6.4 / 6.8, 10240x1536 11.1 / 11.9, 12288x3072 20.5 / 21.4, 16384x3072 26.2 / 21.8; two: 8192x2048
+ * 12.8 / 12.1, 4096x2048 8.0 / 11.3, 4096x8960 27 / 41, Q5 4096x1536 8.0 / 9.3, 4096x896 7.6 / 6.9; three: 4096x1536
+ * 10.8 / 9.4, 2048x1536 6.9 / 9.3, Q5 1024x1536 8.4 / 9.2; four: 2048x2048 7.9 / 11.4, 4096x4864 28.3 / 24.2,
+ * 2048x896 8.0 / 7.0, Q5 1024x1536 9.8 / 9.2, 2048x2048 10.0 / 11.4. */
+bool few_wanted(bool q5, uint32_t nb, uint32_t ntok, uint64_t rows) {
+    const uint32_t passes = (ntok + FEW_NT - 1) / FEW_NT;
+    if (passes > 4 || 16 * passes > nb + 4) return false;
+    if (q5 && nb < 48) return rows * passes <= 4096;
+    return rows * passes <= (passes > 1 ? 8192u : q5 ? 12288u : 16384u);
+}
+
 /* Single launches of many tiles (the LM head: 18992 tiles of 8 rows) run on
  * the pinned persistent kernel; a few thousand tiles fit the device in one
  * wave of workgroups and keep the one-tile-per-workgroup kernel. */
@@ -2623,6 +2799,7 @@ hipError_t launch_typed(MatArgs a, hipStream_t s) {
             }
             return launch_gemv_tile<Q5, FAST>(a, rt, s);
         }
+        if (g_exact_mode == 0 && few_wanted(Q5, a.nb, a.ntok, total_rows)) return launch_few<Q5, FAST>(a, total_rows, s);
         uint32_t tiles = 0, tiles32 = 0;
         for (uint32_t i = 0; i < a.nitems; ++i) {
             a.item[i].tile_begin = tiles;
@@ -2648,16 +2825,27 @@ hipError_t launch_typed(MatArgs a, hipStream_t s) {
          * (0.38) 83.1 / 60.5 / 52.2 / 62.5 */
         const uint64_t w32 = (uint64_t)tiles32 * ((a.ntok + 31) / 32), cu = (uint64_t)cus;
         const bool two_ahead = w32 >= 2 * cu && w32 < 3 * cu;
-        if (g_exact_mode == 1 || (g_exact_mode == 0 && 4 * w32 >= 7 * cu && !two_ahead))
-            return launch_gemm_xm(a, Q5, FAST, 1, s);
-        /* Q8 takes the two-wave split from 5/8 (896x4864 at 192 tokens, W 0.66: 35.4-35.8 / 36.8-37.2 on four
-         * waves), Q5 from 7/8 (1536x8960 at 128 tokens, W 0.75: 66.0-66.5 / 64.1-65.3) */
-        if (g_exact_mode == 3 || (g_exact_mode == 0 && 8 * w32 >= (Q5 ? 7 : 5) * cu))
-            return launch_gemm_xm(a, Q5, FAST, 2, s);
-        if (g_exact_mode == 4 || (g_exact_mode == 0 && 4 * w32 >= cu)) return launch_gemm_xm(a, Q5, FAST, 4, s);
-        /* 8-token tiles where 16-token ones would give fewer than two workgroups per CU (c1 down at 128
+        /* Up to 8 tokens the v_dot4 kernel's 8-token tiles do no work for padding, up to 16 the four-wave split's
+         * 16 x 16 tiles, which lose below W 5/8 to v_dot4 and from W 8 on to the kernels above (8-token v_dot4 / the
+         * bands' choice / four waves at 8 tokens, us: 16384x896 9.8 / 13.0 / 11.3, 131072x896 44.8 / 65.3 / 66.2, Q5
+         * 8960x1536 12.0 / 16.4 / 12.9, 32768x3072 35.4 / 57.6 / 51.9; the bands' / v_dot4 / four waves at 12: 4096x1536
+         * 9.8 / 9.4 / 9.6, 8192x1536 13.6 / 12.9 / 11.3, Q5 16384x3072 37.2 / 33.5 / 29.0, 65536x896 34.1 / 34.3 / 34.1,
+         * 131072x896 66.2 / 68.5 / 72.5) */
+        const bool dot8 = g_exact_mode == 0 && a.ntok <= 8;
+        if (g_exact_mode == 0 && a.ntok > 8 && a.ntok <= 16 && w32 < 8 * cu) {
+            if (8 * w32 >= 5 * cu) return launch_gemm_xm(a, Q5, FAST, 4, s);
+        } else if (!dot8) {
+            if (g_exact_mode == 1 || (g_exact_mode == 0 && 4 * w32 >= 7 * cu && !two_ahead))
+                return launch_gemm_xm(a, Q5, FAST, 1, s);
+            /* Q8 takes the two-wave split from 5/8 (896x4864 at 192 tokens, W 0.66: 35.4-35.8 / 36.8-37.2 on four
+             * waves), Q5 from 7/8 (1536x8960 at 128 tokens, W 0.75: 66.0-66.5 / 64.1-65.3) */
+            if (g_exact_mode == 3 || (g_exact_mode == 0 && 8 * w32 >= (Q5 ? 7 : 5) * cu))
+                return launch_gemm_xm(a, Q5, FAST, 2, s);
+            if (g_exact_mode == 4 || (g_exact_mode == 0 && 4 * w32 >= cu)) return launch_gemm_xm(a, Q5, FAST, 4, s);
+        }
+        /* 8-token tiles also where 16-token ones would give fewer than two workgroups per CU (c1 down at 128
          * tokens: 224 workgroups) */
-        if ((uint64_t)tiles * ((a.ntok + 15) / 16) < 2ull * (uint64_t)cus) {
+        if (a.ntok <= 8 || (uint64_t)tiles * ((a.ntok + 15) / 16) < 2ull * (uint64_t)cus) {
             const uint32_t tok_tiles = (a.ntok + 7) / 8;
             hipLaunchKernelGGL((k_gemm_exact<Q5, FAST, 8>), dim3(tiles * tok_tiles), dim3(WG), 0, s, a, tok_tiles);
         } else {
@@ -2959,6 +3147,7 @@ hipError_t prepare_attention_attributes() {
     const int rows = (int)(((size_t)MAX_ATT_POSITIONS + AR_FIXED) * sizeof(float));
     const int tiled = (int)(((size_t)MAX_ATT_POSITIONS + ATT_SHARED) * sizeof(float));
     const hipError_t es[] = {
+        prepare_few<false, false>(), prepare_few<false, true>(), prepare_few<true, false>(), prepare_few<true, true>(),
         hipFuncSetAttribute((const void *)k_attend_rows<false>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
         hipFuncSetAttribute((const void *)k_attend_rows<true>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
         hipFuncSetAttribute((const void *)k_attend_values<true, AR_HD>, hipFuncAttributeMaxDynamicSharedMemorySize, rows),
