@@ -26,12 +26,21 @@ namespace {
  * the RMSNorm's serial sum), and the prologue's barriers wait for LDS only,
  * so the weight fetch overlaps the activation's quantization. Products, chains
  * and the lane tree are those of k_gemv (exact per-lane order).
+ * A row of one chunk: a thread's task is the same blocks of every tile, so their
+ * activation words, scales and Q5 corrections stay in its registers (read from LDS
+ * per tile they were 32 conflicting words), two tiles' weights are in flight, the
+ * waves take the tiles' chains in turn, and the gated products of up to FU_TILES
+ * tiles are formed together, a thread per row. The RMSNorm, gate/up, SwiGLU and
+ * down projection of Q5 1536 x 8960 29.2 -> 23.6 us, of 2048 x 8192 30.1 -> 23.9,
+ * of Q8 1536 x 8960 28.2 -> 24.8; the RMSNorm's serial sum and the launches of the
+ * quantization and the down projection are most of what is left.
  * ---------------------------------------------------------------------- */
 constexpr int PRO_NORM = 1, PRO_F32 = 2; /* SMQ_ACT_NORM, SMQ_ACT_F32 */
 constexpr uint32_t FU_BATCH = 32; /* activation elements per thread of the widest RMSNorm row */
 static_assert(FU_BATCH * WG == MAX_NORM_K, "the widest RMSNorm row");
 constexpr uint32_t FU_SHORT = 8;  /* elements per thread loaded ahead of the weights (rows up to 2048) */
 constexpr int EPI_STORE = 0, EPI_GLU = 1;
+constexpr uint32_t FU_TILES = 64; /* tiles whose gated products are formed together, a thread per row (RT <= 8) */
 
 /* A workgroup barrier that orders LDS only: this thread's LDS accesses are
  * complete, global loads may stay in flight (s_barrier without the release
@@ -59,6 +68,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
     static_assert(EPI != EPI_GLU || (RT % 2 == 0 && RT * 8 <= 64), "gate/up slots share wave 0");
     __shared__ __attribute__((aligned(16))) float prod[2][(CB / 4) * GS];
     __shared__ __attribute__((aligned(16))) float dsc[FAST ? 2 : 1][FAST ? (CB / 4) * DS : 4];
+    __shared__ float gu[EPI == EPI_GLU ? FU_TILES : 1][RT]; /* gate and up values of a one-chunk row's tiles */
     __shared__ float s_inv;
     __shared__ int s_bad;
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
@@ -102,23 +112,27 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
         }
     };
     const uint32_t nchunks = (nb + CB - 1) / CB;
-    uint32_t wr[NW] = {};
-    auto load_task = [&](const Row &R, uint32_t b) __attribute__((always_inline)) {
-        if (R.ok && b < nb) {
-            const unsigned char *p = R.w + (size_t)b * (Q5 ? Q5_BYTES : Q8_BYTES);
-            const u4a v0 = *(const u4a *)p, v1 = *(const u4a *)(p + 16);
-            wr[0] = v0.x; wr[1] = v0.y; wr[2] = v0.z; wr[3] = v0.w;
-            wr[4] = v1.x; wr[5] = v1.y; wr[6] = v1.z; wr[7] = v1.w;
-            if constexpr (Q5) {
-                const u3a v2 = *(const u3a *)(p + 32);
-                wr[8] = v2.x; wr[9] = v2.y; wr[10] = v2.z;
-            } else {
-                wr[8] = *(const uint32_t *)(p + 32);
-            }
+    uint32_t wr[NW], wn[NW]; /* wn: the second tile of a one-chunk row */
+    auto load_words = [&](const Row &R, uint32_t b, uint32_t (&w)[NW]) __attribute__((always_inline)) {
+        const unsigned char *p = R.w + (size_t)(b < nb ? b : 0) * (Q5 ? Q5_BYTES : Q8_BYTES); /* past the row: not used */
+        const u4a v0 = *(const u4a *)p, v1 = *(const u4a *)(p + 16);
+        w[0] = v0.x; w[1] = v0.y; w[2] = v0.z; w[3] = v0.w;
+        w[4] = v1.x; w[5] = v1.y; w[6] = v1.z; w[7] = v1.w;
+        if constexpr (Q5) {
+            const u3a v2 = *(const u3a *)(p + 32);
+            w[8] = v2.x; w[9] = v2.y; w[10] = v2.z;
+        } else {
+            w[8] = *(const uint32_t *)(p + 32);
         }
     };
+    auto load_task = [&](const Row &R, uint32_t b) __attribute__((always_inline)) { load_words(R, b, wr); };
     Row cur, nxt;
     setup(t0, cur);
+    setup(t0 + 1 < t1 ? t0 + 1 : t0, nxt);
+    auto first_loads = [&]() __attribute__((always_inline)) {
+        load_words(cur, ti * TB, wr);
+        load_words(nxt, ti * TB, wn);
+    };
 
     /* prologue: the activation into LDS. Rows of up to FU_SHORT elements per thread load x (and
      * the norm weights) before the first weight loads are issued: loads complete in order, so
@@ -136,7 +150,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
             if (PRO == PRO_NORM) wv[k] = k < ke && i < n ? a.norm[i] : 0.0f;
         }
     }
-    if (PRO != PRO_NORM) load_task(cur, ti * TB);
+    if (PRO != PRO_NORM) first_loads();
     {
         int bad = 0;
         int8_t *q8 = (int8_t *)act_q;
@@ -181,7 +195,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
                 }
             }
             lds_barrier();
-            load_task(cur, ti * TB); /* after the serial sum (measured faster than before it) */
+            first_loads(); /* after the serial sum (before it: the same time, 23.6 / 23.4 us below) */
             const float inv = s_inv;
             if (tid == 0 && s_bad && a.flag) *a.flag = 1;
             /* (x*inv)*w and its Q8 blocks; uniform: a block's 32 lanes are all below np or past it */
@@ -226,12 +240,98 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
         }
         if (bad && a.flag) *a.flag = 1;
     }
-    if (Q5) {
+    if (Q5 && nchunks > 1) {
         lds_barrier();
         for (uint32_t i = tid; i < nb * 8; i += WG) act_b[i] = dot4(act_q[i], 0xf0f0f0f0u, 0); /* int8 0xf0 = -16 */
     }
     lds_barrier(); /* activation staged */
 
+    auto glu = [&](uint32_t row, float gv, float u) __attribute__((always_inline)) {
+        if (a.flag && (!(fabsf(gv) <= FLT_MAX) || !(fabsf(u) <= FLT_MAX))) *a.flag = 1; /* model.c:309 */
+        float e;
+        if (a.act == 2) {
+            const float g3 = 0.044715f * gv * gv * gv;
+            const float uu = 1.5957691216f * (gv + g3);
+            e = exp_det(-uu);
+        } else {
+            e = exp_det(-gv);
+        }
+        const float den = 1.0f + e;
+        const float sg = gv / den;
+        a.h[row] = u * sg;
+    };
+    if (nchunks == 1) { /* uniform */
+        uint32_t hx[TB][8], hc[TB][8];
+        float hd[TB];
+#pragma unroll
+        for (int k = 0; k < TB; ++k) {
+            const uint32_t b = ti * TB + k < nb ? ti * TB + k : k;
+            hd[k] = act_d[b];
+#pragma unroll
+            for (int l = 0; l < 8; ++l) {
+                hx[k][l] = act_q[b * 8 + l];
+                hc[k][l] = Q5 ? dot4(hx[k][l], 0xf0f0f0f0u, 0) : 0; /* int8 0xf0 = -16 */
+            }
+        }
+        auto one = [&](uint32_t tile, uint32_t (&w)[NW]) __attribute__((always_inline)) {
+            const uint32_t j = tile - t0;
+            float *pb = prod[j & 1u];
+            Q5Fields f[2];
+            if (Q5) q5_parse_pair(w, f[0], f[1]);
+            float d[TB];
+#pragma unroll
+            for (int k = 0; k < TB; ++k) {
+                d[k] = (Q5 ? f[k].scale : __uint_as_float(w[0])) * hd[k];
+                if (FAST) dsc[j & 1u][((ti * TB + k) / 4) * DS + tr * 4 + ((ti * TB + k) % 4)] = d[k];
+            }
+            float *slot = tile_slot<GS>(pb, tr, ti * TB);
+#pragma unroll
+            for (int l = 0; l < 8; ++l) {
+                float v[TB];
+#pragma unroll
+                for (int k = 0; k < TB; ++k) {
+                    const int sv = Q5 ? dot4(q5_codes(f[k], l), hx[k][l], hc[k][l]) : dot4(w[1 + l], hx[k][l], 0);
+                    v[k] = FAST ? (float)sv : d[k] * (float)sv;
+                }
+                put_lane<TB>(slot, l, v[0], v[TB - 1]);
+            }
+            Row R;
+            setup(tile + 2 < t1 ? tile + 2 : t1 - 1, R);
+            load_words(R, ti * TB, w); /* consumed: two tiles ahead in flight */
+            lds_barrier();
+            if (tid / 64 == (j & 3u)) { /* the waves take the tiles' chains in turn */
+                const uint32_t slot8 = tid & 63u; /* row slot8 / 8, lane slot8 % 8 */
+                float acc = 0.0f;
+                if (slot8 < RT * 8)
+                    chain_sum<FAST, CB / 4>(acc, (const float4 *)pb + slot8, GS / 4,
+                                            FAST ? (const float4 *)dsc[j & 1u] + slot8 / 8 : nullptr, DS / 4, nb);
+                const float v = reduce8_to_lane7(acc);
+                if ((slot8 & 7) == 7 && slot8 < RT * 8) {
+                    if (EPI == EPI_GLU) {
+                        gu[j % FU_TILES][slot8 / 8] = v;
+                    } else {
+                        Row C;
+                        setup(tile, C);
+                        const Item &I = a.item[C.item];
+                        const uint32_t r = C.r0 + slot8 / 8;
+                        if (r < I.rows) store_out(I, a.flag, 0, r, v);
+                    }
+                }
+            }
+            if (EPI == EPI_GLU && (j % FU_TILES == FU_TILES - 1 || tile + 1 == t1)) { /* uniform */
+                lds_barrier();
+                constexpr uint32_t half = RT / 2 > 0 ? RT / 2 : 1;
+                const uint32_t base = j / FU_TILES * FU_TILES, i = tid / half, row = (t0 + base + i) * half + tid % half;
+                if (i <= j - base && row < a.rows) glu(row, gu[i][tid % half], gu[i][half + tid % half]);
+                lds_barrier();
+            }
+        };
+        for (uint32_t tile = t0; tile < t1; tile += 2) {
+            one(tile, wr);
+            if (tile + 1 < t1) one(tile + 1, wn); /* uniform */
+        }
+        return;
+    }
     uint32_t step = 0; /* products buffer parity */
     for (uint32_t tile = t0; tile < t1; ++tile) {
         if (tile + 1 < t1) setup(tile + 1, nxt);
@@ -277,21 +377,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
                 const float v = reduce8_to_lane7(acc);
                 const float u = __shfl_down(v, RT * 4, 64); /* up slot tr + RT/2 */
                 const uint32_t row = tile * (RT / 2 > 0 ? RT / 2 : 1) + tid / 8;
-                if ((tid & 7) == 7 && tid < RT * 4 && row < a.rows) {
-                    const float gv = v;
-                    if (a.flag && (!(fabsf(gv) <= FLT_MAX) || !(fabsf(u) <= FLT_MAX))) *a.flag = 1; /* model.c:309 */
-                    float e;
-                    if (a.act == 2) {
-                        const float g3 = 0.044715f * gv * gv * gv;
-                        const float uu = 1.5957691216f * (gv + g3);
-                        e = exp_det(-uu);
-                    } else {
-                        e = exp_det(-gv);
-                    }
-                    const float den = 1.0f + e;
-                    const float sg = gv / den;
-                    a.h[row] = u * sg;
-                }
+                if ((tid & 7) == 7 && tid < RT * 4 && row < a.rows) glu(row, v, u);
             }
         } else if (tid < RT * 8) {
             const float v = reduce8_to_lane7(acc);
