@@ -15,8 +15,8 @@
  * 128 adds 281 ns; 128 v_mul and 128 v_add 231 ns, but 342 ns when the common
  * operand comes by DPP, and scalar loads of it did not keep up.
  * 256 tokens at positions 3328-3583, 12 heads of 128 over 2 KV heads: 4220 us
- * with a workgroup per token, head and 32 columns -> 176 us (scores 72,
- * softmax 35, values 88; the products and adds alone need about 46 + 46 at
+ * with a workgroup per token, head and 32 columns -> 171 us (scores 72,
+ * softmax 30, values 88; the products and adds alone need about 46 + 46 at
  * four waves per SIMD, and this many rows fill less than two). */
 #include "smq_device.h"
 
@@ -234,6 +234,7 @@ __global__ __launch_bounds__(64 * AP_ROWS) void k_ap_softmax(PreArgs a) {
         return;
     }
     float t = 0.0f;
+    __builtin_amdgcn_s_setprio(3); /* the chain before the three waves of its SIMD that form weights: 177 -> 171 us above */
     __syncthreads();
     for (uint32_t c = 0; c < nch; ++c) { /* chunk c, while the others form chunk c + 1 */
         const uint32_t left = groups - c * CG, n = left < CG ? left : CG;
