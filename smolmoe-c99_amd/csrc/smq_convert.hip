@@ -11,11 +11,10 @@
  * are packed as 16 nibble bytes (element j low, j + 16 high) after the f16
  * scale and the 32-bit plane of fifth bits (docs/FORMAT.md:124-134).
  *
- * Mapping: a workgroup takes 24 consecutive blocks. Half a wave per block finds the
- * extreme; then a lane per (block, candidate), 504 of them in two rounds over the 256
- * threads, runs the binary64 sum over the block's elements in LDS; one lane per block
- * picks the winner; half a wave per block quantizes and packs into LDS, and the 528
- * bytes go out as words.
+ * Mapping: a wave takes six consecutive blocks and needs no barrier. Eight lanes per block
+ * load four elements each and find the extreme; then a lane per (block, candidate), 63 of
+ * them in each of two rounds, sums over the block's elements in LDS; eight lanes per block
+ * quantize and pack, and the 132 bytes go out as words.
  *
  * What bounds it is the 21 x 32 terms per block, so a term is as short as its value
  * allows. q * d is exact in binary32 (5 and 11 significant bits). x - q * d is exact too:
@@ -24,9 +23,16 @@
  * a subnormal half. For |q| = 1, rint gave 1, so p = fl(x * dinv) is at least 1/2 + 2^-24
  * and, with both roundings below 2^-24, x / d at least 1/2 (1 - 2^-48): as x and d / 2 are
  * binary32 numbers, x >= d / 2. The square of a binary32 number is exact in binary64, so
- * one fused multiply-add is the reference's square, then sum. A term is four binary32
- * operations, a conversion and that fma. 8960 x 1536: 253.4 us with half a wave per block (21 of 32 lanes) and four
- * binary64 operations a term -> 71.2 us.
+ * one fused multiply-add is the reference's square, then sum.
+ *
+ * The sums are formed in binary32 first: 32 fused steps of terms >= 0 are within 2^-19 of the
+ * exact sum, so a candidate more than a factor 1 + 2^-17 above the smallest is not the minimum
+ * (below 2^-99, where a square may underflow, all are kept). Only where another candidate is
+ * within that are the kept ones summed in binary64; one block in some thousand of N(0, s).
+ * A term is five binary32 operations, which at full rate take 37 us of 8960 x 1536. Measured
+ * there: half a wave per block and four binary64 operations a term 253 us; a workgroup per 24
+ * blocks, a conversion and a binary64 fma a term 71.2; binary32 sums 67.6; a wave per six blocks
+ * 63.1; the winner's scale from its lane, scalar row division, no half operands 55.4.
  */
 #include <float.h>
 
@@ -37,9 +43,9 @@ namespace smq {
 namespace {
 
 constexpr uint32_t CV_WG = 256;
-constexpr uint32_t CV_BLOCKS = 24; /* 21 candidates of each: 504 lanes of two rounds */
+constexpr uint32_t CV_BLOCKS = 6; /* per wave: 21 candidates of each are 126 lanes of two rounds */
 constexpr uint32_t CV_K = 21;
-constexpr uint32_t CV_PITCH = 36; /* floats per block: a wave's three or four blocks on distinct banks */
+constexpr uint32_t CV_PITCH = 36; /* floats per block: a round's three blocks on distinct banks */
 
 /* lrintf(v * inv) clamped to the 5-bit range (kernels.c:1064-1067). A NaN product takes
  * -16: x86-64's lrintf returns LONG_MIN for it (cvtss2si's "integer indefinite"), which the
@@ -63,105 +69,190 @@ __device__ __forceinline__ uint32_t q5_candidate(float extreme, uint32_t k) {
     return to_half_bits(extreme / divisor);
 }
 
+/* LDS written by this wave's lanes, read by its other lanes (LDS serves a wave in order). */
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t or_dpp(uint32_t v) {
+    return v | (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+}
+
+/* quad: rows of whole quads of elements at 16-byte addresses (one read per lane). */
 __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t blocks, uint32_t nb, uint32_t cols,
-                                                       unsigned char *out) {
-    __shared__ __attribute__((aligned(16))) float xs[CV_BLOCKS * CV_PITCH];
-    __shared__ double errs[CV_BLOCKS * CV_K];
-    __shared__ float ext[CV_BLOCKS], winv[CV_BLOCKS];
-    __shared__ uint32_t whalf[CV_BLOCKS];
-    __shared__ __attribute__((aligned(4))) unsigned char bytes[CV_BLOCKS * Q5_BYTES];
-    const uint32_t tid = threadIdx.x, j = tid % 32, b0 = blockIdx.x * CV_BLOCKS;
-    constexpr uint32_t U = CV_BLOCKS * 32 / CV_WG;
-    float v[U];
-    bool valid[U];
+                                                       bool quad, unsigned char *out) {
+    constexpr uint32_t W = CV_WG / 64;
+    __shared__ __attribute__((aligned(16))) float s_x[W][CV_BLOCKS * CV_PITCH];
+    __shared__ double s_exact[W][CV_BLOCKS * CV_K];
+    __shared__ float s_scale[W][CV_BLOCKS][2];
+    __shared__ unsigned long long s_best[W][CV_BLOCKS]; /* bits of the smallest sum, then its candidate */
+    __shared__ __attribute__((aligned(4))) unsigned char s_bytes[W][CV_BLOCKS * Q5_BYTES];
+    const uint32_t L = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint64_t first = ((uint64_t)blockIdx.x * W + w) * CV_BLOCKS;
+    if (first >= blocks) return; /* no barrier below */
+    const uint32_t b0 = (uint32_t)first, slot = L / 8, t = L % 8;
+    float *xs = s_x[w];
+    double *exact = s_exact[w];
+    unsigned long long *best = s_best[w];
+    unsigned char *bytes = s_bytes[w];
+
+    const uint32_t blk = b0 + slot;
+    uint32_t row = b0 / nb, col = b0 - row * nb + slot; /* scalar, then this lane's block */
+    if (nb >= 8) { /* slot < 8: at most one row further */
+        row += col >= nb;
+        col -= col >= nb ? nb : 0;
+    } else {
+        row += col / nb;
+        col %= nb;
+    }
+    const uint32_t c = col * 32 + 4 * t;
+    const bool live = slot < CV_BLOCKS && blk < blocks;
+    const float *src = x + (size_t)row * cols + c;
+    f4v v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (quad) {
+        if (live && c < cols) v = *(const f4v *)src;
+    } else {
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-        const uint32_t blk = b0 + u * (CV_WG / 32) + tid / 32, row = blk / nb, c = (blk - row * nb) * 32 + j;
-        valid[u] = blk < blocks && c < cols;
-        v[u] = valid[u] ? x[(size_t)row * cols + c] : 0.0f;
+        for (uint32_t i = 0; i < 4; ++i)
+            if (live && c + i < cols) v[i] = src[i];
     }
     /* the signed extreme: largest |x|, first on ties (kernels.c:1090-1091); a NaN never wins
      * (fabsf(NaN) > m is false there), so it enters as -1 and an all-NaN block keeps extreme 0 */
+    float m = -1.0f, own = 0.0f;
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-        const uint32_t slot = u * (CV_WG / 32) + tid / 32;
-        xs[slot * CV_PITCH + j] = v[u];
-        const float av = v[u] == v[u] ? fabsf(v[u]) : -1.0f, m = max32(av);
-        const uint64_t at = __ballot(av == m);
-        const uint32_t first = (uint32_t)__builtin_ctz((uint32_t)((tid & 63u) < 32 ? at : at >> 32));
-        const float e = __shfl(v[u], (int)first, 32);
-        if (j == 0) ext[slot] = m > 0.0f ? e : 0.0f;
+    for (uint32_t i = 0; i < 4; ++i) {
+        const float av = fabsf(v[i]);
+        own = av > m ? v[i] : own;
+        m = av > m ? av : m;
     }
-    __syncthreads();
+    float m8 = m, o = dpp_f<0xB1>(m8); /* the block's eight lanes */
+    m8 = o > m8 ? o : m8;
+    o = dpp_f<0x4E>(m8);
+    m8 = o > m8 ? o : m8;
+    o = dpp_f<0x141>(m8);
+    m8 = o > m8 ? o : m8;
+    const uint32_t at = (uint32_t)(__ballot(m == m8) >> (8 * slot)) & 255u;
+    const float e8 = __shfl(own, (int)(8 * slot + (uint32_t)__builtin_ctz(at | 256u)), 64);
+    const float extreme8 = m8 > 0.0f ? e8 : 0.0f; /* this lane's block's */
+    if (slot < CV_BLOCKS) *(f4v *)&xs[slot * CV_PITCH + 4 * t] = v;
+    if (L < CV_BLOCKS) best[L] = ~0ull;
+    wave_sync();
 
-    /* error sums in element order (a NaN element makes every kept candidate's sum NaN; the zeros past a
-     * short block's end add zeros) */
-    for (uint32_t id = tid; id < CV_BLOCKS * CV_K; id += CV_WG) {
-        const uint32_t slot = id / CV_K, k = id - slot * CV_K;
-        const float extreme = ext[slot];
-        double err = -1.0; /* skipped: no sum of squares is -1 */
-        const float d = half_to_float(q5_candidate(extreme, k));
-        if (extreme != 0.0f && d != 0.0f && fabsf(d) <= FLT_MAX) {
-            const float dinv = 1.0f / d;
-            const float4 *x4 = (const float4 *)&xs[slot * CV_PITCH];
+    auto diff = [&](float e, float d, float dinv) __attribute__((always_inline)) {
+        const float q = __builtin_amdgcn_fmed3f(__builtin_rintf(e * dinv), -16.0f, 15.0f);
+        return __builtin_fmaf(-q, d, e);
+    };
+    /* the sums in binary32 (a NaN element makes every kept candidate's sum NaN; the zeros past a short
+     * block's end add zeros), then the first minimum over the kept candidates, as
+     * `best < 0 || err < best` (kernels.c:1099): the first kept one is taken whatever its error, so NaN sums
+     * leave the first kept candidate */
+    const uint32_t kb = L / CV_K, k = L - kb * CV_K; /* lane 63: no candidate */
+    float err[2], dk[2], ik[2]; /* sum, scale and its inverse */
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) {
+        const uint32_t s = 3 * r + (kb < 3 ? kb : 2);
+        const float extreme = __shfl(extreme8, (int)(8 * s), 64);
+        float d = half_to_float(q5_candidate(extreme, k));
+        asm("" : "+v"(d)); /* a binary32 register, not a half operand of every fma */
+        const bool kept = kb < 3 && extreme != 0.0f && d != 0.0f && fabsf(d) <= FLT_MAX;
+        const float dinv = 1.0f / d;
+        float acc = 0.0f;
+        const f4v *x4 = (const f4v *)&xs[s * CV_PITCH];
+#pragma unroll
+        for (uint32_t g = 0; g < 8; ++g) {
+            const f4v xv = x4[g];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const float de = diff(xv[i], d, dinv);
+                acc = __builtin_fmaf(de, de, acc);
+            }
+        }
+        err[r] = kept ? acc : -1.0f; /* skipped: no sum of squares is -1 */
+        dk[r] = d;
+        ik[r] = dinv;
+        const uint32_t bits = acc == acc ? __float_as_uint(acc) : 0x7fc00000u;
+        if (kept) atomicMin(&best[s], (unsigned long long)bits << 32 | k);
+    }
+    wave_sync();
+    bool near[2], close = false;
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) {
+        const unsigned long long key = best[3 * r + (kb < 3 ? kb : 2)];
+        const float wide = __uint_as_float((uint32_t)(key >> 32)) * (1.0f + 0x1p-17f), lim = wide < 0x1p-99f ? 0x1p-99f : wide;
+        near[r] = err[r] >= 0.0f && err[r] <= lim;
+        close |= near[r] && k != (uint32_t)key;
+    }
+    if (__ballot(close)) { /* uniform: in element order, as the reference sums */
+#pragma unroll
+        for (uint32_t r = 0; r < 2; ++r) {
+            const uint32_t s = 3 * r + (kb < 3 ? kb : 2);
             double acc = 0.0;
-#pragma unroll
-            for (uint32_t g = 0; g < 8; ++g) {
-                const float4 xv = x4[g];
-                const float e4[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) {
-                    const float q = __builtin_amdgcn_fmed3f(__builtin_rintf(e4[i] * dinv), -16.0f, 15.0f);
-                    const double de = (double)__builtin_fmaf(-q, d, e4[i]);
-                    acc = __builtin_fma(de, de, acc);
+#pragma unroll 8
+            for (uint32_t i = 0; i < 32; ++i) {
+                const double de = (double)diff(xs[s * CV_PITCH + i], dk[r], ik[r]);
+                acc = __builtin_fma(de, de, acc);
+            }
+            if (kb < 3) exact[s * CV_K + k] = near[r] ? acc : -1.0;
+        }
+        wave_sync();
+        if (L < CV_BLOCKS) {
+            double low = -1.0;
+            uint32_t win = CV_K;
+            for (uint32_t i = 0; i < CV_K; ++i) {
+                const double e = exact[L * CV_K + i];
+                if (e != -1.0 && (low < 0.0 || e < low)) {
+                    low = e;
+                    win = i;
                 }
             }
-            err = acc;
+            if (win < CV_K) best[L] = win;
         }
-        errs[id] = err;
+        wave_sync();
     }
-    __syncthreads();
-    /* first minimum over the kept candidates, as `best < 0 || err < best` (kernels.c:1099): the
-     * first kept one is taken whatever its error, so NaN sums leave the first kept candidate */
-    if (tid < CV_BLOCKS) {
-        uint32_t win = CV_K;
-        double best = -1.0;
-#pragma unroll
-        for (uint32_t k = 0; k < CV_K; ++k) {
-            const double e = errs[tid * CV_K + k];
-            if (e != -1.0 && (best < 0.0 || e < best)) {
-                best = e;
-                win = k;
-            }
-        }
-        const uint32_t h = win < CV_K ? q5_candidate(ext[tid], win) : 0u;
-        whalf[tid] = h;
-        winv[tid] = win < CV_K ? 1.0f / half_to_float(h) : 0.0f; /* 0: no scale was kept */
-    }
-    __syncthreads();
 
     /* pack: high plane bit j = bit 4 of code j; byte 6 + j (j < 16) = code j | code j+16 << 4 */
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-        const uint32_t slot = u * (CV_WG / 32) + tid / 32;
-        const float inv = winv[slot];
-        const uint32_t q = (uint32_t)((valid[u] && inv != 0.0f ? q5_level(v[u], inv) : 0) + 16);
-        const uint64_t hb = __ballot((q >> 4) & 1u);
-        const uint32_t high = (uint32_t)((tid & 63u) < 32 ? hb : hb >> 32), half = whalf[slot];
-        const uint32_t upper = __shfl_down(q, 16, 32);
-        unsigned char *o = bytes + slot * Q5_BYTES;
-        if (j < 16) o[6 + j] = (unsigned char)((q & 15u) | ((upper & 15u) << 4));
-        else if (j < 18) o[j - 16] = (unsigned char)(half >> (8 * (j - 16)));
-        else if (j < 22) o[2 + (j - 18)] = (unsigned char)(high >> (8 * (j - 18)));
+    for (uint32_t r = 0; r < 2; ++r) { /* the winner's lane leaves its scale and inverse */
+        const uint32_t s = 3 * r + kb;
+        if (kb < 3 && k == (uint32_t)best[s]) {
+            s_scale[w][s][0] = dk[r];
+            s_scale[w][s][1] = ik[r];
+        }
     }
-    __syncthreads();
-    const uint32_t live = (blocks - b0 < CV_BLOCKS ? blocks - b0 : CV_BLOCKS) * Q5_BYTES;
-    unsigned char *o = out + (size_t)b0 * Q5_BYTES;
-    if (((uintptr_t)out & 3u) == 0) { /* b0 * 22 is a multiple of 528 */
-        if (tid < live / 4) ((uint32_t *)o)[tid] = ((const uint32_t *)bytes)[tid];
-        else if (tid == live / 4 && live % 4) *(uint16_t *)(o + (live & ~3u)) = *(const uint16_t *)(bytes + (live & ~3u));
+    wave_sync();
+    const bool won = slot < CV_BLOCKS && (uint32_t)best[slot] < CV_K; /* else no scale was kept */
+    const uint32_t ss = slot < CV_BLOCKS ? slot : 0;
+    const float inv = won ? s_scale[w][ss][1] : 0.0f;
+    const uint32_t half = won ? to_half_bits(s_scale[w][ss][0]) : 0u;
+    uint32_t low = 0, high = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t q = (uint32_t)((c + i < cols && inv != 0.0f ? q5_level(v[i], inv) : 0) + 16);
+        low |= (q & 15u) << (8 * i);
+        high |= (q >> 4) << (4 * t + i);
+    }
+    high = or_dpp<0x141>(or_dpp<0x4E>(or_dpp<0xB1>(high)));
+    const uint32_t word = low | __shfl_down(low, 4, 8) << 4; /* of lanes 0-3 */
+    if (slot < CV_BLOCKS) {
+        uint16_t *o16 = (uint16_t *)(bytes + slot * Q5_BYTES);
+        if (t < 4) {
+            o16[3 + 2 * t] = (uint16_t)word;
+            o16[4 + 2 * t] = (uint16_t)(word >> 16);
+        } else if (t == 4) {
+            o16[0] = (uint16_t)half;
+        } else if (t < 7) {
+            o16[t - 4] = (uint16_t)(high >> (16 * (t - 5)));
+        }
+    }
+    wave_sync();
+    const uint32_t n = (blocks - b0 < CV_BLOCKS ? blocks - b0 : CV_BLOCKS) * Q5_BYTES;
+    unsigned char *dst = out + (size_t)b0 * Q5_BYTES;
+    if (((uintptr_t)out & 3u) == 0) { /* b0 * 22 is a multiple of 132 */
+        if (L < n / 4) ((uint32_t *)dst)[L] = ((const uint32_t *)bytes)[L];
+        else if (L == n / 4 && n % 4) *(uint16_t *)(dst + (n & ~3u)) = *(const uint16_t *)(bytes + (n & ~3u));
     } else {
-        for (uint32_t i = tid; i < live; i += CV_WG) o[i] = bytes[i];
+        for (uint32_t i = L; i < n; i += 64) dst[i] = bytes[i];
     }
 }
 
@@ -170,10 +261,12 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
 hipError_t launch_quantize_q5(const float *x, uint32_t rows, uint32_t cols, unsigned char *out, hipStream_t s) {
     const uint64_t blocks = (uint64_t)rows * ((cols + 31) / 32);
     if (!blocks) return hipSuccess;
-    const uint64_t grid = (blocks + CV_BLOCKS - 1) / CV_BLOCKS;
-    if (blocks > 0xffffffffu - CV_BLOCKS) return hipErrorInvalidValue; /* more than the device memory holds */
+    constexpr uint32_t per = CV_BLOCKS * (CV_WG / 64);
+    const uint64_t grid = (blocks + per - 1) / per;
+    const bool quad = cols % 4 == 0 && ((uintptr_t)x & 15u) == 0;
+    if (blocks > 0xffffffffu - per) return hipErrorInvalidValue; /* more than the device memory holds */
     hipLaunchKernelGGL(k_quantize_q5, dim3((uint32_t)grid), dim3(CV_WG), 0, s, x, (uint32_t)blocks, (cols + 31) / 32, cols,
-                       out);
+                       quad, out);
     return hipGetLastError();
 }
 

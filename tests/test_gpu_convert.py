@@ -145,3 +145,18 @@ def test_half_steps(orc):
         x[r] = (steps.view(np.int32) + rng.integers(-3, 4, 64)).astype(np.int32).view(np.float32)
         x[r, ::32] = np.float32(rng.uniform(14.5, 16.5)) * d * (1 if r % 2 else -1)
     check(orc, x, "half steps")
+
+
+def test_close_sums(orc):
+    """Candidates whose error sums tie or differ by less than binary32 tells: rows on the 5-bit grid (a zero sum) and
+    an ulp off it, scales at the smallest halves (several candidates round to one), at every place of a wave's blocks."""
+    rng = np.random.default_rng(63)
+    x = np.zeros((384, 224), np.float32)
+    for r in range(384):
+        d = np.float32(np.float16(rng.uniform(1.0, 2.0) * 2.0 ** int(rng.integers(-23, 4))))
+        q = rng.integers(-16, 16, 224)
+        q[rng.integers(0, 32)::32] = -16
+        x[r] = q * d
+        if r % 3:
+            x[r] = (x[r].view(np.int32) + (rng.integers(0, 40, 224) == 0) * (r % 3)).astype(np.int32).view(np.float32)
+    check(orc, x, "close sums")
