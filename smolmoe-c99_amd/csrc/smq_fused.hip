@@ -300,6 +300,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
             load_words(R, ti * TB, w); /* consumed: two tiles ahead in flight */
             lds_barrier();
             if (tid / 64 == (j & 3u)) { /* the waves take the tiles' chains in turn */
+                __builtin_amdgcn_s_setprio(2); /* before the products of its SIMD's other waves: 24.1 -> 23.6 us above */
                 const uint32_t slot8 = tid & 63u; /* row slot8 / 8, lane slot8 % 8 */
                 float acc = 0.0f;
                 if (slot8 < RT * 8)
@@ -317,6 +318,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
                         if (r < I.rows) store_out(I, a.flag, 0, r, v);
                     }
                 }
+                __builtin_amdgcn_s_setprio(0);
             }
             if (EPI == EPI_GLU && (j % FU_TILES == FU_TILES - 1 || tile + 1 == t1)) { /* uniform */
                 lds_barrier();
