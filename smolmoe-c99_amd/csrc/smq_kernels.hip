@@ -1758,8 +1758,6 @@ __device__ __forceinline__ float att_long(const float *sc, float *prod, uint32_t
         load(vb, AL_VP);
         put(va, 0, 0);
         load(va, 2 * AL_VP);
-    } else {
-        __builtin_amdgcn_s_setprio(3); /* before the products of the wave on its SIMD: 12 heads of 128 at 3072 26.3 -> 26.2 us */
     }
     __syncthreads();
     auto step = [&](uint32_t p0, uint32_t b, f4v (&v)[AL_VL]) __attribute__((always_inline)) {
@@ -1814,7 +1812,7 @@ __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uin
     const float inv = *s_inv;
 
     float o = 0.0f;
-    if (np > AR_VP) { /* uniform */
+    if (__builtin_expect(np > AR_VP, 0)) { /* uniform; its code after the short path's */
         o = att_long<ROPE>(sc, prod, np, last, inv, vbase, vrope, kvd);
     } else {
 #pragma unroll
