@@ -1782,10 +1782,15 @@ __device__ __forceinline__ float att_long(const float *sc, float *prod, uint32_t
  * (order-free, NaN never wins as in softmax_inv, kernels.c:1146-1148),
  * exp_det(s - max) in parallel, the total in position order by one lane,
  * then the products (s_p*inv)*v_p[j] to LDS and lane j's sum of its column in
- * position order (kernels.c:1165); past AR_VP positions by att_long. pre holds
- * the value rows (up to AR_VP positions). The 32 outputs go to
+ * position order (kernels.c:1165); LONG, past AR_VP positions, by att_long. pre
+ * holds the value rows (not LONG). A kernel branches on np between two whole
+ * copies, the long one placed last: in a decode step, where each kernel runs
+ * cold after five others, one copy with both value paths cost 32 tokens at 512
+ * positions 25,310 us against 25,190 without the long path, two copies 25,065 (back
+ * to back the three tie), and a call of the long path was 2 % slower at 3001
+ * positions. The 32 outputs go to
  * out[0, 32); with xd, their Q8 block to *xd / xq[0, 32) (kernels.c:912-935). */
-template <bool ROPE>
+template <bool ROPE, bool LONG>
 __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uint32_t np, uint32_t last,
                                          float4 (&pre)[AR_VL], const float *vbase, const float *vrope,
                                          uint32_t kvd, uint32_t vrow, uint32_t vcol, const uint64_t *etab,
@@ -1812,7 +1817,7 @@ __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uin
     const float inv = *s_inv;
 
     float o = 0.0f;
-    if (__builtin_expect(np > AR_VP, 0)) { /* uniform; its code after the short path's */
+    if constexpr (LONG) {
         o = att_long<ROPE>(sc, prod, np, last, inv, vbase, vrope, kvd);
     } else {
 #pragma unroll
@@ -1955,9 +1960,12 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
     }
 
     const uint32_t nbq = sh.q_dim / QK, blk = (h * AR_HD + j0) / QK;
-    att_tail<ROPE>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red,
-                   &s_inv, att + (size_t)t * sh.q_dim + (size_t)h * AR_HD + j0, xd ? xd + (size_t)t * nbq + blk : nullptr,
-                   xq ? xq + ((size_t)t * nbq + blk) * QK : nullptr, flag);
+    float *out = att + (size_t)t * sh.q_dim + (size_t)h * AR_HD + j0, *xdb = xd ? xd + (size_t)t * nbq + blk : nullptr;
+    int8_t *xqb = xq ? xq + ((size_t)t * nbq + blk) * QK : nullptr;
+    if (__builtin_expect(np <= AR_VP, 1)) /* uniform */
+        att_tail<ROPE, false>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, &s_inv, out, xdb, xqb, flag);
+    else
+        att_tail<ROPE, true>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, &s_inv, out, xdb, xqb, flag);
 }
 
 /* Decode attention in two launches (one token, head_dim 64): the K rows are
@@ -2117,32 +2125,15 @@ __global__ __launch_bounds__(AS_WG) void k_attend_scores_hd(const float *q, cons
 /* k_attend_values: workgroup (head, 32 coordinates) loads its scores row and
  * its value rows up front, then steps 2-4 of the row attention (att_tail). HD: the
  * head size, or 0 for a multiple of 32 read at run time. */
-template <bool ROPE, uint32_t HD>
-__global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_attend_values(
-    const float *vcache, float *att, AttnShape sh, uint32_t pos0, const int32_t *pos_dev, float *xd, int8_t *xq,
-    const float *vraw, const float *scores, int *flag) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    __shared__ uint64_t etab[32];
-    __shared__ float red[AR_WG / 64];
-    __shared__ float s_inv;
-    const uint32_t hd = HD ? HD : sh.head_dim, ngrp = hd / ATT_JW;
-    const uint32_t tid = threadIdx.x, g = blockIdx.x % ngrp, h = blockIdx.x / ngrp;
-    const uint32_t kh = h / (sh.heads / sh.kv_heads), kvd = sh.kv_dim, j0 = g * ATT_JW;
-    const uint32_t pos = pos_dev ? (uint32_t)*pos_dev : pos0;
-    if (pos >= sh.context) return; /* flagged by the scores launch */
-    const uint32_t start = sh.window && pos >= sh.window ? pos - sh.window + 1 : 0, np = pos - start + 1;
-    const uint32_t last = np - 1;
-    float *sc = lds;
-    float *prod = lds + ((sh.context + 3) & ~3u);
-    const float *vbase = vcache + (size_t)start * kvd + (size_t)kh * hd + j0;
-    const float *vrope = ROPE ? vraw + (size_t)kh * hd + j0 : nullptr;
-    const float *srow = scores + (size_t)h * sh.context;
-    const uint32_t vrow = tid / (ATT_JW / 4), vcol = (tid % (ATT_JW / 4)) * 4;
-
+template <bool ROPE, bool LONG>
+__device__ __forceinline__ void att_values(const float *srow, float *sc, float *prod, uint32_t np, const float *vbase,
+                                           const float *vrope, uint32_t kvd, uint64_t *etab, float *red, float *s_inv,
+                                           float *out, float *xd, int8_t *xq, int *flag) {
+    const uint32_t tid = threadIdx.x, last = np - 1, vrow = tid / (ATT_JW / 4), vcol = (tid % (ATT_JW / 4)) * 4;
     /* issue order = need order: the table, the scores (a round of AR_WG x AS_LD), the first value rows */
     uint64_t ev = 0;
     if (tid < 32) ev = EXP2_TABLE[tid];
-    constexpr uint32_t AS_LD = 4;
+    constexpr uint32_t AS_LD = LONG ? 4 : (AR_VP + AR_WG - 1) / AR_WG;
     float sv[AS_LD];
 #pragma unroll
     for (uint32_t u = 0; u < AS_LD; ++u) {
@@ -2150,7 +2141,7 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
         sv[u] = p < np ? srow[p] : 0.0f;
     }
     float4 pre[AR_VL];
-    if (np <= AR_VP) att_load_values<ROPE>(pre, vbase, vrope, kvd, 0, np, last, vrow, vcol); /* uniform */
+    if constexpr (!LONG) att_load_values<ROPE>(pre, vbase, vrope, kvd, 0, np, last, vrow, vcol);
     if (tid < 32) etab[tid] = ev;
     float high = -FLT_MAX;
 #pragma unroll
@@ -2161,14 +2152,41 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
             high = sv[u] > high ? sv[u] : high;
         }
     }
-    for (uint32_t p = tid + AS_LD * AR_WG; p < np; p += AR_WG) { /* long contexts */
-        const float v = srow[p];
-        sc[p] = v;
-        high = v > high ? v : high;
-    }
+    if constexpr (LONG)
+        for (uint32_t p = tid + AS_LD * AR_WG; p < np; p += AR_WG) {
+            const float v = srow[p];
+            sc[p] = v;
+            high = v > high ? v : high;
+        }
+    att_tail<ROPE, LONG>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, s_inv, out, xd, xq, flag);
+}
+
+template <bool ROPE, uint32_t HD>
+__global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_attend_values(
+    const float *vcache, float *att, AttnShape sh, uint32_t pos0, const int32_t *pos_dev, float *xd, int8_t *xq,
+    const float *vraw, const float *scores, int *flag) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ uint64_t etab[32];
+    __shared__ float red[AR_WG / 64];
+    __shared__ float s_inv;
+    const uint32_t hd = HD ? HD : sh.head_dim, ngrp = hd / ATT_JW;
+    const uint32_t g = blockIdx.x % ngrp, h = blockIdx.x / ngrp;
+    const uint32_t kh = h / (sh.heads / sh.kv_heads), kvd = sh.kv_dim, j0 = g * ATT_JW;
+    const uint32_t pos = pos_dev ? (uint32_t)*pos_dev : pos0;
+    if (pos >= sh.context) return; /* flagged by the scores launch */
+    const uint32_t start = sh.window && pos >= sh.window ? pos - sh.window + 1 : 0, np = pos - start + 1;
+    float *sc = lds;
+    float *prod = lds + ((sh.context + 3) & ~3u);
+    const float *vbase = vcache + (size_t)start * kvd + (size_t)kh * hd + j0;
+    const float *vrope = ROPE ? vraw + (size_t)kh * hd + j0 : nullptr;
+    const float *srow = scores + (size_t)h * sh.context;
     const uint32_t blk = (h * hd + j0) / QK;
-    att_tail<ROPE>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, &s_inv,
-                   att + (size_t)h * hd + j0, xd ? xd + blk : nullptr, xq ? xq + (size_t)blk * QK : nullptr, flag);
+    float *out = att + (size_t)h * hd + j0, *xdb = xd ? xd + blk : nullptr;
+    int8_t *xqb = xq ? xq + (size_t)blk * QK : nullptr;
+    if (__builtin_expect(np <= AR_VP, 1)) /* uniform */
+        att_values<ROPE, false>(srow, sc, prod, np, vbase, vrope, kvd, etab, red, &s_inv, out, xdb, xqb, flag);
+    else
+        att_values<ROPE, true>(srow, sc, prod, np, vbase, vrope, kvd, etab, red, &s_inv, out, xdb, xqb, flag);
 }
 
 /* Prefill attention (many tokens, head_dim 64): workgroup (token, KV head)
