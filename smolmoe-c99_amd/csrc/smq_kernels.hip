@@ -1784,11 +1784,10 @@ __device__ __forceinline__ float att_long(const float *sc, float *prod, uint32_t
  * then the products (s_p*inv)*v_p[j] to LDS and lane j's sum of its column in
  * position order (kernels.c:1165); LONG, past AR_VP positions, by att_long. pre
  * holds the value rows (not LONG). A kernel branches on np between two whole
- * copies, the long one placed last: in a decode step, where each kernel runs
- * cold after five others, one copy with both value paths cost 32 tokens at 512
- * positions 25,310 us against 25,190 without the long path, two copies 25,065 (back
- * to back the three tie), and a call of the long path was 2 % slower at 3001
- * positions. The 32 outputs go to
+ * copies: in a decode step, where each kernel runs cold after five others, one
+ * copy with both value paths cost 32 tokens at 512 positions 25,310 us against
+ * 25,190 without the long path, two copies 24,980 (back to back the three tie),
+ * and a call of the long path was 2 % slower at 3001 positions. The 32 outputs go to
  * out[0, 32); with xd, their Q8 block to *xd / xq[0, 32) (kernels.c:912-935). */
 template <bool ROPE, bool LONG>
 __device__ __forceinline__ void att_tail(float high, float *sc, float *prod, uint32_t np, uint32_t last,
@@ -1962,7 +1961,7 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
     const uint32_t nbq = sh.q_dim / QK, blk = (h * AR_HD + j0) / QK;
     float *out = att + (size_t)t * sh.q_dim + (size_t)h * AR_HD + j0, *xdb = xd ? xd + (size_t)t * nbq + blk : nullptr;
     int8_t *xqb = xq ? xq + ((size_t)t * nbq + blk) * QK : nullptr;
-    if (__builtin_expect(np <= AR_VP, 1)) /* uniform */
+    if (np <= AR_VP) /* uniform */
         att_tail<ROPE, false>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, &s_inv, out, xdb, xqb, flag);
     else
         att_tail<ROPE, true>(high, sc, prod, np, last, pre, vbase, vrope, kvd, vrow, vcol, etab, red, &s_inv, out, xdb, xqb, flag);
@@ -2183,7 +2182,7 @@ __global__ __launch_bounds__(AR_WG) __attribute__((amdgpu_waves_per_eu(1, 2))) v
     const uint32_t blk = (h * hd + j0) / QK;
     float *out = att + (size_t)h * hd + j0, *xdb = xd ? xd + blk : nullptr;
     int8_t *xqb = xq ? xq + (size_t)blk * QK : nullptr;
-    if (__builtin_expect(np <= AR_VP, 1)) /* uniform */
+    if (np <= AR_VP) /* uniform */
         att_values<ROPE, false>(srow, sc, prod, np, vbase, vrope, kvd, etab, red, &s_inv, out, xdb, xqb, flag);
     else
         att_values<ROPE, true>(srow, sc, prod, np, vbase, vrope, kvd, etab, red, &s_inv, out, xdb, xqb, flag);
