@@ -3089,18 +3089,29 @@ bool attention_decode_split(const AttnShape &sh, const void *q, const void *kcac
 
 /* Whether a prefill's attention is faster in 16-row tiles (three launches, each position's adds of a row in one
  * wave) than a workgroup per token and KV head or per token, head and 32 columns (one launch, the adds of a
- * column split from its products). Measured on MI355X, us, tiles / the other:
- * k_attend_group's shapes by the positions seen: 512 tokens from 0 44.7 / 46.4, 400 from 0 36.3 / 34.4, 512 from
- * 512 72 / 99, 2 from 1000 36 / 47, 2 from 256 20.2 / 18.2.
+ * column split from its products). Both sides as costs in ns, fitted to 500 shapes on MI355X.
+ * k_attend_group runs about 6 us and 18 ns per position and 4 more per query head of a group, as long as 400
+ * workgroups of a token and KV head are resident; the tiles 13 us, 25 ns per position and 6 ns per 1000 positions and
+ * query heads. Measured, us, tiles / group: 14 heads of 64 over 2 KV heads, 512 tokens from 0 44.7 / 46.4, 400 from 0
+ * 36.3 / 34.4, 512 from 512 72 / 99, 2 from 1000 36 / 47, 2 from 256 20.2 / 18.2; 9 over 3, 17 from 564 with a window
+ * of 512 28.3 / 20.6, 16 from 572 27.3 / 23.4; 32 over 8, 61 from 718 with that window 34.1 / 29.8, 89 from 202
+ * 24.8 / 33.6.
  * The others run about 4 us and 14 (head_dim 128: 26) ns per position in each round of one workgroup per CU,
- * the tiles 13 us and 25 ns per position while few: 14 heads of 64, 16 tokens from 3800 107 / 112, from 1000
- * 38 / 33, 64 from 0 16 / 34, 256 from 0 23 / 146; 12 heads of 128, 2 from 3000 87 / 81, 8 from 3000 88 / 156,
- * 4 from 500 27 / 17, 8 from 500 28 / 33. */
+ * the tiles 13 us and 25 ns per position while few; against k_attend_rows (3 us and 14.5 ns a round) the tiles count
+ * 16 us and 22 ns: 14 heads of 64, 16 tokens from 3800 107 / 112, from 1000 38 / 33, 64 from 0 16 / 34, 256 from 0
+ * 23 / 146, 22 from 331 with a window of 128 18.4 / 16.3; 9 heads of 64, 40 from 3276 with that window 20.1 / 16.4;
+ * 12 heads of 128, 2 from 3000 87 / 81, 8 from 3000 88 / 156, 4 from 500 27 / 17, 8 from 500 28 / 33. */
 bool attend_tiles_wanted(const AttnShape &sh, uint32_t ntok, uint32_t pos0) {
     uint64_t seen = (uint64_t)pos0 + ntok;
     if (sh.window && sh.window + (uint64_t)ntok < seen) seen = sh.window + (uint64_t)ntok;
-    if (sh.head_dim == AR_HD && sh.context <= AG_MAXP && sh.heads / sh.kv_heads <= AG_MAXG) return seen >= 512;
+    const bool rows = sh.head_dim == AR_HD;
+    const uint32_t grp = sh.heads / sh.kv_heads;
+    if (rows && sh.context <= AG_MAXP && grp <= AG_MAXG) {
+        const uint64_t groups = (uint64_t)ntok * sh.kv_heads, load = groups > 400 ? groups : 400;
+        return (6000 + (18 + 4 * grp) * seen) * load / 400 > 13000 + 25 * seen + 6 * (uint64_t)ntok * sh.heads * seen / 1000;
+    }
     const uint64_t wgs = (uint64_t)ntok * sh.heads * ((sh.head_dim + ATT_JW - 1) / ATT_JW), rounds = (wgs + 255) / 256;
+    if (rows) return rounds * (6000 + 29 * seen) > 2 * (16000 + 22 * seen);
     return rounds * (4000 + (sh.head_dim <= AR_HD ? 14 : 26) * seen) > 13000 + 25 * seen;
 }
 
