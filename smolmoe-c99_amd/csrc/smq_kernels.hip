@@ -2642,7 +2642,7 @@ hipError_t launch_few(MatArgs a, uint32_t total_rows, hipStream_t s) {
  * 2048x896 8.0 / 7.0, Q5 1024x1536 9.8 / 9.2, 2048x2048 10.0 / 11.4. */
 bool few_wanted(bool q5, uint32_t nb, uint32_t ntok, uint64_t rows) {
     const uint32_t passes = (ntok + FEW_NT - 1) / FEW_NT;
-    if (passes > 4 || 16 * passes > nb + 4) return false;
+    if (passes > 4 || 16 * passes > nb + 4 || (nb < 16 && rows * passes > 2048)) return false;
     if (q5 && nb < 48) return rows * passes <= 4096;
     return rows * passes <= (passes > 1 ? 8192u : q5 ? 12288u : 16384u);
 }
@@ -2843,14 +2843,19 @@ hipError_t launch_typed(MatArgs a, hipStream_t s) {
         const uint64_t w32 = (uint64_t)tiles32 * ((a.ntok + 31) / 32), cu = (uint64_t)cus;
         const bool two_ahead = w32 >= 2 * cu && w32 < 3 * cu;
         /* Up to 8 tokens the v_dot4 kernel's 8-token tiles do no work for padding, up to 16 the four-wave split's
-         * 16 x 16 tiles, which lose below W 5/8 to v_dot4 and from W 8 on to the kernels above (8-token v_dot4 / the
+         * 16 x 16 tiles, which lose to v_dot4 while its two 8-token workgroups per 32 rows take one round (W up to 1/2; to
+         * 5/8 for rows of at most 12 blocks) and from W 8 on (rows under 28 blocks: 7/4) to 32 x 32 tiles (8-token v_dot4 / the
          * bands' choice / four waves at 8 tokens, us: 16384x896 9.8 / 13.0 / 11.3, 131072x896 44.8 / 65.3 / 66.2, Q5
-         * 8960x1536 12.0 / 16.4 / 12.9, 32768x3072 35.4 / 57.6 / 51.9; the bands' / v_dot4 / four waves at 12: 4096x1536
-         * 9.8 / 9.4 / 9.6, 8192x1536 13.6 / 12.9 / 11.3, Q5 16384x3072 37.2 / 33.5 / 29.0, 65536x896 34.1 / 34.3 / 34.1,
-         * 131072x896 66.2 / 68.5 / 72.5) */
+         * 8960x1536 12.0 / 16.4 / 12.9, 32768x3072 35.4 / 57.6 / 51.9; the bands' / v_dot4 / four waves at 12: 8192x1536
+         * 13.6 / 12.9 / 11.3, Q5 16384x3072 37.2 / 33.5 / 29.0, 65536x896 34.1 / 34.3 / 34.1, 131072x896 66.2 / 68.5 /
+         * 72.5; v_dot4 / four waves at 9, weights streamed: 4096x1536 9.5 / 9.8, 4128x1536 11.9 / 10.6, 4864x896 9.0 /
+         * 8.0, 4096x4864 24.5 / 25.0, 4128x4864 32.2 / 28.3, Q5 4096x2048 11.5 / 12.0, 4128x2048 14.5 / 13.3, 4864x128
+         * 3.7 / 4.3, 4128x384 4.7 / 4.9; 32 x 32 / four waves at 16: 14336x576 9.4 / 10.0, 24576x576 12.4 / 14.6, Q5
+         * 32768x256 7.9 / 10.3) */
         const bool dot8 = g_exact_mode == 0 && a.ntok <= 8;
         if (g_exact_mode == 0 && a.ntok > 8 && a.ntok <= 16 && w32 < 8 * cu) {
-            if (8 * w32 >= 5 * cu) return launch_gemm_xm(a, Q5, FAST, 4, s);
+            if (a.nb < 28 && 4 * w32 >= 7 * cu) return launch_gemm_xm(a, Q5, FAST, 1, s);
+            if (a.nb > 12 ? 2 * w32 > cu : 8 * w32 >= 5 * cu) return launch_gemm_xm(a, Q5, FAST, 4, s);
         } else if (!dot8) {
             if (g_exact_mode == 1 || (g_exact_mode == 0 && 4 * w32 >= 7 * cu && !two_ahead))
                 return launch_gemm_xm(a, Q5, FAST, 1, s);
