@@ -11,10 +11,11 @@
  * are packed as 16 nibble bytes (element j low, j + 16 high) after the f16
  * scale and the 32-bit plane of fifth bits (docs/FORMAT.md:124-134).
  *
- * Mapping: a wave takes six consecutive blocks and needs no barrier. Eight lanes per block
- * load four elements each and find the extreme; then a lane per (block, candidate), 63 of
- * them in each of two rounds, sums over the block's elements in LDS; eight lanes per block
- * quantize and pack, and the 132 bytes go out as words.
+ * Mapping: a wave takes six (few blocks in all: three) consecutive blocks and needs no
+ * barrier. Eight lanes per block load four elements each and find the extreme; then a lane
+ * per (block, candidate), 63 of them in each of two rounds (one), sums over the block's
+ * elements in LDS; eight lanes per block quantize and pack, and the bytes go out as words
+ * (half words: three blocks are 66 bytes).
  *
  * What bounds it is the 21 x 32 terms per block, so a term is as short as its value
  * allows. q * d is exact in binary32 (5 and 11 significant bits). x - q * d is exact too:
@@ -43,7 +44,6 @@ namespace smq {
 namespace {
 
 constexpr uint32_t CV_WG = 256;
-constexpr uint32_t CV_BLOCKS = 6; /* per wave: 21 candidates of each are 126 lanes of two rounds */
 constexpr uint32_t CV_K = 21;
 constexpr uint32_t CV_PITCH = 36; /* floats per block: a round's three blocks on distinct banks */
 
@@ -79,10 +79,12 @@ __device__ __forceinline__ uint32_t or_dpp(uint32_t v) {
     return v | (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
 }
 
-/* quad: rows of whole quads of elements at 16-byte addresses (one read per lane). */
+/* quad: rows of whole quads of elements at 16-byte addresses (one read per lane). ROUNDS: one of 63 candidates a wave
+ * where the blocks leave the chip idle, so that a wave's serial chain is half as long. */
+template <uint32_t ROUNDS>
 __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t blocks, uint32_t nb, uint32_t cols,
                                                        bool quad, unsigned char *out) {
-    constexpr uint32_t W = CV_WG / 64;
+    constexpr uint32_t W = CV_WG / 64, CV_BLOCKS = 3 * ROUNDS; /* per wave: 21 candidates of three blocks a round */
     __shared__ __attribute__((aligned(16))) float s_x[W][CV_BLOCKS * CV_PITCH];
     __shared__ double s_exact[W][CV_BLOCKS * CV_K];
     __shared__ float s_scale[W][CV_BLOCKS][2];
@@ -91,13 +93,12 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
     const uint32_t L = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint64_t first = ((uint64_t)blockIdx.x * W + w) * CV_BLOCKS;
     if (first >= blocks) return; /* no barrier below */
-    const uint32_t b0 = (uint32_t)first, slot = L / 8, t = L % 8;
+    const uint32_t b0 = (uint32_t)first, left = blocks - b0, slot = L / 8, t = L % 8;
     float *xs = s_x[w];
     double *exact = s_exact[w];
     unsigned long long *best = s_best[w];
     unsigned char *bytes = s_bytes[w];
 
-    const uint32_t blk = b0 + slot;
     uint32_t row = b0 / nb, col = b0 - row * nb + slot; /* scalar, then this lane's block */
     if (nb >= 8) { /* slot < 8: at most one row further */
         row += col >= nb;
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
         col %= nb;
     }
     const uint32_t c = col * 32 + 4 * t;
-    const bool live = slot < CV_BLOCKS && blk < blocks;
+    const bool live = slot < CV_BLOCKS && slot < left;
     const float *src = x + (size_t)row * cols + c;
     f4v v = {0.0f, 0.0f, 0.0f, 0.0f};
     if (quad) {
@@ -148,9 +149,9 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
      * `best < 0 || err < best` (kernels.c:1099): the first kept one is taken whatever its error, so NaN sums
      * leave the first kept candidate */
     const uint32_t kb = L / CV_K, k = L - kb * CV_K; /* lane 63: no candidate */
-    float err[2], dk[2], ik[2]; /* sum, scale and its inverse */
+    float err[ROUNDS], dk[ROUNDS], ik[ROUNDS]; /* sum, scale and its inverse */
 #pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) {
+    for (uint32_t r = 0; r < ROUNDS; ++r) {
         const uint32_t s = 3 * r + (kb < 3 ? kb : 2);
         const float extreme = __shfl(extreme8, (int)(8 * s), 64);
         float d = half_to_float(q5_candidate(extreme, k));
@@ -175,9 +176,9 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
         if (kept) atomicMin(&best[s], (unsigned long long)bits << 32 | k);
     }
     wave_sync();
-    bool near[2], close = false;
+    bool near[ROUNDS], close = false;
 #pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) {
+    for (uint32_t r = 0; r < ROUNDS; ++r) {
         const unsigned long long key = best[3 * r + (kb < 3 ? kb : 2)];
         const float wide = __uint_as_float((uint32_t)(key >> 32)) * (1.0f + 0x1p-17f), lim = wide < 0x1p-99f ? 0x1p-99f : wide;
         near[r] = err[r] >= 0.0f && err[r] <= lim;
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
     }
     if (__ballot(close)) { /* uniform: in element order, as the reference sums */
 #pragma unroll
-        for (uint32_t r = 0; r < 2; ++r) {
+        for (uint32_t r = 0; r < ROUNDS; ++r) {
             const uint32_t s = 3 * r + (kb < 3 ? kb : 2);
             double acc = 0.0;
 #pragma unroll 8
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
 
     /* pack: high plane bit j = bit 4 of code j; byte 6 + j (j < 16) = code j | code j+16 << 4 */
 #pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) { /* the winner's lane leaves its scale and inverse */
+    for (uint32_t r = 0; r < ROUNDS; ++r) { /* the winner's lane leaves its scale and inverse */
         const uint32_t s = 3 * r + kb;
         if (kb < 3 && k == (uint32_t)best[s]) {
             s_scale[w][s][0] = dk[r];
@@ -246,11 +247,13 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
         }
     }
     wave_sync();
-    const uint32_t n = (blocks - b0 < CV_BLOCKS ? blocks - b0 : CV_BLOCKS) * Q5_BYTES;
+    const uint32_t n = (left < CV_BLOCKS ? left : CV_BLOCKS) * Q5_BYTES;
     unsigned char *dst = out + (size_t)b0 * Q5_BYTES;
-    if (((uintptr_t)out & 3u) == 0) { /* b0 * 22 is a multiple of 132 */
+    if (ROUNDS == 2 && ((uintptr_t)out & 3u) == 0) { /* b0 * 22 is a multiple of 132 */
         if (L < n / 4) ((uint32_t *)dst)[L] = ((const uint32_t *)bytes)[L];
         else if (L == n / 4 && n % 4) *(uint16_t *)(dst + (n & ~3u)) = *(const uint16_t *)(bytes + (n & ~3u));
+    } else if (ROUNDS == 1 && ((uintptr_t)out & 1u) == 0) { /* 66 bytes */
+        if (L < n / 2) ((uint16_t *)dst)[L] = ((const uint16_t *)bytes)[L];
     } else {
         for (uint32_t i = L; i < n; i += 64) dst[i] = bytes[i];
     }
@@ -258,16 +261,23 @@ __global__ __launch_bounds__(CV_WG) void k_quantize_q5(const float *x, uint32_t 
 
 }  // namespace
 
+template <uint32_t ROUNDS>
+static hipError_t launch_q5_rounds(const float *x, uint32_t blocks, uint32_t cols, bool quad, unsigned char *out, hipStream_t s) {
+    constexpr uint32_t per = 3 * ROUNDS * (CV_WG / 64);
+    hipLaunchKernelGGL(k_quantize_q5<ROUNDS>, dim3((uint32_t)(((uint64_t)blocks + per - 1) / per)), dim3(CV_WG), 0, s, x, blocks,
+                       (cols + 31) / 32, cols, quad, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_quantize_q5(const float *x, uint32_t rows, uint32_t cols, unsigned char *out, hipStream_t s) {
     const uint64_t blocks = (uint64_t)rows * ((cols + 31) / 32);
     if (!blocks) return hipSuccess;
-    constexpr uint32_t per = CV_BLOCKS * (CV_WG / 64);
-    const uint64_t grid = (blocks + per - 1) / per;
     const bool quad = cols % 4 == 0 && ((uintptr_t)x & 15u) == 0;
-    if (blocks > 0xffffffffu - per) return hipErrorInvalidValue; /* more than the device memory holds */
-    hipLaunchKernelGGL(k_quantize_q5, dim3((uint32_t)grid), dim3(CV_WG), 0, s, x, (uint32_t)blocks, (cols + 31) / 32, cols,
-                       quad, out);
-    return hipGetLastError();
+    if (blocks > 0xffffffffu) return hipErrorInvalidValue; /* more than the device memory holds */
+    /* one round while about four such waves per SIMD hold every block. Measured on MI355X (us, one round / two): 1 block
+     * 2.8 / 3.3, 500 4.3 / 5.3, 5000 4.7 / 5.6, 20000 6.5 / 7.0, 30000 8.25 / 8.2, 50000 11.2 / 10.1 */
+    if (blocks <= 28000) return launch_q5_rounds<1>(x, (uint32_t)blocks, cols, quad, out, s);
+    return launch_q5_rounds<2>(x, (uint32_t)blocks, cols, quad, out, s);
 }
 
 }  // namespace smq

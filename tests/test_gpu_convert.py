@@ -90,6 +90,13 @@ def test_edge_rows(orc, request):
             assert np.array_equal(got[0], ref.quantize_q5_row(x[i])), f"edge row {i} vs reference"
 
 
+def test_edge_rows_two_rounds(orc):
+    """The edge rows among enough blocks for two rounds a wave, each at every place of a wave's six blocks."""
+    x = np.tile(edge_rows(), (430, 1))
+    assert x.shape[0] * 3 > 28000
+    check(orc, x[1:], "edges in two rounds")
+
+
 @pytest.mark.parametrize("cols", [1, 7, 31, 32, 33, 45, 63, 65, 1000])
 def test_partial_blocks(orc, cols):
     """Widths with a partial last block: padding never enters the extreme or the error, codes 16."""
@@ -120,9 +127,12 @@ def test_round_trip_bound(orc):
         assert np.all(np.abs(y - x[r]) <= scales * 1.0001 + 1e-7)
 
 
-@pytest.mark.parametrize("rows,cols,offset", [(1, 1, 0), (25, 31, 0), (7, 33, 0), (3, 1000, 2), (5, 773, 1), (49, 64, 0)])
+@pytest.mark.parametrize("rows,cols,offset", [(1, 1, 0), (25, 31, 0), (7, 33, 0), (3, 1000, 2), (5, 773, 1), (49, 64, 0),
+                                              (28000, 31, 0), (28001, 31, 0), (14001, 33, 2), (9335, 77, 1),
+                                              (3501, 250, 0)])
 def test_block_groups(orc, rows, cols, offset):
-    """24 blocks per workgroup: partial groups, rows that end inside one, short blocks, outputs at any byte."""
+    """12 blocks per workgroup, 24 past 28000 blocks: partial groups, rows that end inside one, short blocks, outputs at
+    any byte."""
     say("q5 block groups", rows, cols, offset)
     x = synth.normal(61, rows * cols, 1.0).reshape(rows, cols)
     n = rows * ((cols + 31) // 32) * 22
