@@ -26,14 +26,16 @@ namespace {
  * the RMSNorm's serial sum), and the prologue's barriers wait for LDS only,
  * so the weight fetch overlaps the activation's quantization. Products, chains
  * and the lane tree are those of k_gemv (exact per-lane order).
- * A row of one chunk: a thread's task is the same blocks of every tile, so their
+ * ONE, a row of one chunk: a thread's task is the same blocks of every tile, so their
  * activation words, scales and Q5 corrections stay in its registers (read from LDS
  * per tile they were 32 conflicting words), two tiles' weights are in flight, the
  * waves take the tiles' chains in turn, and the gated products of up to FU_TILES
  * tiles are formed together, a thread per row. The RMSNorm, gate/up, SwiGLU and
  * down projection of Q5 1536 x 8960 29.2 -> 23.6 us, of 2048 x 8192 30.1 -> 23.9,
  * of Q8 1536 x 8960 28.2 -> 24.8; the RMSNorm's serial sum and the launches of the
- * quantization and the down projection are most of what is left.
+ * quantization and the down projection are most of what is left. An instantiation
+ * of its own: beside the general form its registers cost both of them workgroups per
+ * CU (Q8 gate/up rows of 8 tiles 97 registers, apart 88 and 80).
  * ---------------------------------------------------------------------- */
 constexpr int PRO_NORM = 1, PRO_F32 = 2; /* SMQ_ACT_NORM, SMQ_ACT_F32 */
 constexpr uint32_t FU_BATCH = 32; /* activation elements per thread of the widest RMSNorm row */
@@ -57,8 +59,10 @@ __device__ __forceinline__ uint32_t find_fused_item(const FusedArgs &a, uint32_t
     return it;
 }
 
-template <bool Q5, bool FAST, int RT, int PRO, int EPI>
-__global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles) {
+template <bool Q5, bool FAST, int RT, int PRO, int EPI, bool ONE>
+/* the general Q8 form at 8 rows: one register past the next workgroup per CU without the bound */
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(!Q5 && !ONE && RT == 8 ? (EPI == EPI_GLU ? 6 : 7) : 1, 8))) void
+k_gemv_fused(FusedArgs a, uint32_t ntiles) {
     constexpr int TB = Q5 ? 2 : 1;    /* blocks per task */
     constexpr int TPR = WG / RT;      /* tasks per row per chunk */
     constexpr int CB = TPR * TB;      /* blocks per chunk */
@@ -68,7 +72,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
     static_assert(EPI != EPI_GLU || (RT % 2 == 0 && RT * 8 <= 64), "gate/up slots share wave 0");
     __shared__ __attribute__((aligned(16))) float prod[2][(CB / 4) * GS];
     __shared__ __attribute__((aligned(16))) float dsc[FAST ? 2 : 1][FAST ? (CB / 4) * DS : 4];
-    __shared__ float gu[EPI == EPI_GLU ? FU_TILES : 1][RT]; /* gate and up values of a one-chunk row's tiles */
+    __shared__ float gu[ONE && EPI == EPI_GLU ? FU_TILES : 1][RT]; /* gate and up values of the tiles */
     __shared__ float s_inv;
     __shared__ int s_bad;
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
@@ -112,9 +116,10 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
         }
     };
     const uint32_t nchunks = (nb + CB - 1) / CB;
-    uint32_t wr[NW], wn[NW]; /* wn: the second tile of a one-chunk row */
+    uint32_t wr[NW], wn[ONE ? NW : 1]; /* wn: the second tile of a one-chunk row */
     auto load_words = [&](const Row &R, uint32_t b, uint32_t (&w)[NW]) __attribute__((always_inline)) {
-        const unsigned char *p = R.w + (size_t)(b < nb ? b : 0) * (Q5 ? Q5_BYTES : Q8_BYTES); /* past the row: not used */
+        if (!ONE && !(R.ok && b < nb)) return;
+        const unsigned char *p = R.w + (size_t)(!ONE || b < nb ? b : 0) * (Q5 ? Q5_BYTES : Q8_BYTES); /* past the row: not used */
         const u4a v0 = *(const u4a *)p, v1 = *(const u4a *)(p + 16);
         w[0] = v0.x; w[1] = v0.y; w[2] = v0.z; w[3] = v0.w;
         w[4] = v1.x; w[5] = v1.y; w[6] = v1.z; w[7] = v1.w;
@@ -128,10 +133,12 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
     auto load_task = [&](const Row &R, uint32_t b) __attribute__((always_inline)) { load_words(R, b, wr); };
     Row cur, nxt;
     setup(t0, cur);
-    setup(t0 + 1 < t1 ? t0 + 1 : t0, nxt);
     auto first_loads = [&]() __attribute__((always_inline)) {
         load_words(cur, ti * TB, wr);
-        load_words(nxt, ti * TB, wn);
+        if constexpr (ONE) {
+            setup(t0 + 1 < t1 ? t0 + 1 : t0, nxt);
+            load_words(nxt, ti * TB, wn);
+        }
     };
 
     /* prologue: the activation into LDS. Rows of up to FU_SHORT elements per thread load x (and
@@ -240,7 +247,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
         }
         if (bad && a.flag) *a.flag = 1;
     }
-    if (Q5 && nchunks > 1) {
+    if (Q5 && !ONE) {
         lds_barrier();
         for (uint32_t i = tid; i < nb * 8; i += WG) act_b[i] = dot4(act_q[i], 0xf0f0f0f0u, 0); /* int8 0xf0 = -16 */
     }
@@ -260,7 +267,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
         const float sg = gv / den;
         a.h[row] = u * sg;
     };
-    if (nchunks == 1) { /* uniform */
+    if constexpr (ONE) {
         uint32_t hx[TB][8], hc[TB][8];
         float hd[TB];
 #pragma unroll
@@ -332,8 +339,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
             one(tile, wr);
             if (tile + 1 < t1) one(tile + 1, wn); /* uniform */
         }
-        return;
-    }
+    } else {
     uint32_t step = 0; /* products buffer parity */
     for (uint32_t tile = t0; tile < t1; ++tile) {
         if (tile + 1 < t1) setup(tile + 1, nxt);
@@ -389,6 +395,7 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
         }
         cur = nxt;
     }
+    }
 }
 
 /* Dynamic LDS limit of every k_gemv_fused instance, raised once at smq_init (before any
@@ -396,6 +403,35 @@ __global__ __launch_bounds__(WG) void k_gemv_fused(FusedArgs a, uint32_t ntiles)
  * MAX_FAST_NB Q5 blocks of 17 floats. */
 constexpr size_t FUSED_MAX_LDS = (3 * (size_t)MAX_NORM_K + (size_t)MAX_FAST_NB * 17u) * 4u;
 static_assert(FUSED_MAX_LDS <= 160u * 1024u, "within one CU's LDS");
+
+/* The workgroups that are resident at once, at most: each takes a range of tiles, so the prologue runs once per
+ * workgroup (the occupancy of an instantiation is read at the widest LDS seen). */
+template <bool Q5, int RT, int PRO, int EPI, bool ONE>
+hipError_t fused_resident(size_t lds, uint32_t &out) {
+    static size_t queried_lds = 0;
+    static int resident = 0, cus = 0;
+    if (lds > queried_lds) {
+        int per_cu = 0, dev = 0;
+        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gemv_fused<Q5, false, RT, PRO, EPI, ONE>,
+                                                                    WG, lds);
+        if (e == hipSuccess) e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e != hipSuccess) return e;
+        resident = (per_cu > 0 ? per_cu : 1) * (cus > 0 ? cus : 1);
+        queried_lds = lds;
+    }
+    out = (uint32_t)resident;
+    /* more than four per CU only repeat the prologue: Q8 576 -> 7168, us, four / five per CU 8.75 / 9.2 */
+    if (ONE && EPI == EPI_GLU && cus > 0 && out > 4 * (uint32_t)cus) out = 4 * (uint32_t)cus;
+    return hipSuccess;
+}
+
+template <bool Q5, int RT, int PRO, int EPI, bool ONE>
+hipError_t launch_fused_form(const FusedArgs &a, uint32_t tiles, uint32_t resident, size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL((k_gemv_fused<Q5, false, RT, PRO, EPI, ONE>), dim3(tiles < resident ? tiles : resident), dim3(WG), lds, s,
+                       a, tiles);
+    return hipGetLastError();
+}
 
 template <bool Q5, int RT, int PRO, int EPI>
 hipError_t launch_fused_rt(FusedArgs a, hipStream_t s) {
@@ -412,34 +448,38 @@ hipError_t launch_fused_rt(FusedArgs a, hipStream_t s) {
     if (!tiles) return hipSuccess;
     const size_t lds = ((PRO == PRO_NORM ? 3 * ((a.n + 3) / 4 * 4) : 0) + (size_t)a.nb * (Q5 ? 17u : 9u)) * 4u;
     if (lds > FUSED_MAX_LDS) return hipErrorInvalidValue; /* past the limit prepare_fused_attributes set */
-    /* at most one resident wave of workgroups, each taking a range of tiles: the prologue runs
-     * once per workgroup (the occupancy of this instantiation is read at the widest LDS seen) */
-    static size_t queried_lds = 0;
-    static int resident = 0;
-    if (lds > queried_lds) {
-        int per_cu = 0, dev = 0, cus = 0;
-        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gemv_fused<Q5, false, RT, PRO, EPI>,
-                                                                    WG, lds);
-        if (e == hipSuccess) e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    uint32_t resident = 0;
+    if (a.nb <= (uint32_t)(WG / RT * (Q5 ? 2 : 1))) { /* one chunk */
+        /* Q8 rows of up to 32 blocks while the general form gives each workgroup one tile: nothing is reused then, and
+         * more of its workgroups are resident (gate/up, us, general / one chunk: 256 -> 4096 6.1 / 6.7, 896 -> 2560 8.7 /
+         * 9.1; 576 -> 8960, several tiles each, 10.8 / 9.3) */
+        constexpr bool lone = !Q5 && RT == 8;
+        hipError_t e = lone ? fused_resident<Q5, RT, PRO, EPI, false>(lds, resident) : hipSuccess;
         if (e != hipSuccess) return e;
-        resident = (per_cu > 0 ? per_cu : 1) * (cus > 0 ? cus : 1);
-        queried_lds = lds;
+        if (!lone || tiles > resident) {
+            e = fused_resident<Q5, RT, PRO, EPI, true>(lds, resident);
+            return e != hipSuccess ? e : launch_fused_form<Q5, RT, PRO, EPI, true>(a, tiles, resident, lds, s);
+        }
     }
-    const uint32_t grid = tiles < (uint32_t)resident ? tiles : (uint32_t)resident;
-    hipLaunchKernelGGL((k_gemv_fused<Q5, false, RT, PRO, EPI>), dim3(grid), dim3(WG), lds, s, a, tiles);
-    return hipGetLastError();
+    const hipError_t e = fused_resident<Q5, RT, PRO, EPI, false>(lds, resident);
+    return e != hipSuccess ? e : launch_fused_form<Q5, RT, PRO, EPI, false>(a, tiles, resident, lds, s);
 }
 
-template <bool Q5, int RT, int PRO, int EPI>
-hipError_t raise_fused_lds() { /* at most what the CU holds beside the kernel's static LDS */
-    const void *fn = (const void *)k_gemv_fused<Q5, false, RT, PRO, EPI>;
+template <bool Q5, int RT, int PRO, int EPI, bool ONE>
+hipError_t raise_fused_form() { /* at most what the CU holds beside the kernel's static LDS */
+    const void *fn = (const void *)k_gemv_fused<Q5, false, RT, PRO, EPI, ONE>;
     hipFuncAttributes at;
     const hipError_t e = hipFuncGetAttributes(&at, fn);
     if (e != hipSuccess) return e;
     const size_t room = (size_t)160 * 1024 - at.sharedSizeBytes;
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)(FUSED_MAX_LDS < room ? FUSED_MAX_LDS : room));
+}
+
+template <bool Q5, int RT, int PRO, int EPI>
+hipError_t raise_fused_lds() {
+    const hipError_t e = raise_fused_form<Q5, RT, PRO, EPI, false>();
+    return e != hipSuccess ? e : raise_fused_form<Q5, RT, PRO, EPI, true>();
 }
 
 template <bool Q5>

@@ -2634,12 +2634,12 @@ hipError_t launch_few(MatArgs a, uint32_t total_rows, hipStream_t s) {
 }
 /* Where k_gemv_few beats the tiles of k_gemm_exact and k_gemm_xm, by its passes of four tokens: a row of about 16
  * blocks per pass, and rows x passes up to 8192 (Q5 rows under 48 blocks, which leave tasks of its one chunk idle,
- * 4096); one pass up to 16384 rows (Q5 12288). Measured on MI355X (us, k_gemv_few / the best tile kernel): one pass:
- * 16384x896 9.4 / 9.7, 24576x896 12.4 / 11.9, 16384x3072 18.6 / 23.0, 32768x3072 38.4 / 37.2, Q5 8192x896 8.7 / 6.8,
- * 4096x896 6.4 / 6.8, 10240x1536 11.1 / 11.9, 12288x3072 20.5 / 21.4, 16384x3072 26.2 / 21.8; two: 8192x2048
- * 12.8 / 12.1, 4096x2048 8.0 / 11.3, 4096x8960 27 / 41, Q5 4096x1536 8.0 / 9.3, 4096x896 7.6 / 6.9; three: 4096x1536
- * 10.8 / 9.4, 2048x1536 6.9 / 9.3, Q5 1024x1536 8.4 / 9.2; four: 2048x2048 7.9 / 11.4, 4096x4864 28.3 / 24.2,
- * 2048x896 8.0 / 7.0, Q5 1024x1536 9.8 / 9.2, 2048x2048 10.0 / 11.4. */
+ * 4096; rows under 16 blocks 2048); one pass up to 16384 rows (Q5 12288). Measured on MI355X (us, k_gemv_few / the best
+ * tile kernel): one pass: 16384x896 9.4 / 9.7, 24576x896 12.4 / 11.9, 16384x3072 18.6 / 23.0, 32768x3072 38.4 / 37.2, Q5
+ * 8192x896 8.7 / 6.8, 4096x896 6.4 / 6.8, 10240x1536 11.1 / 11.9, 12288x3072 20.5 / 21.4, 16384x3072 26.2 / 21.8,
+ * 2688x448 5.6 / 4.85, Q5 4.9 / 4.2; two: 8192x2048 12.8 / 12.1, 4096x2048 8.0 / 11.3, 4096x8960 27 / 41, Q5 4096x1536
+ * 8.0 / 9.3, 4096x896 7.6 / 6.9; three: 4096x1536 10.8 / 9.4, 2048x1536 6.9 / 9.3, Q5 1024x1536 8.4 / 9.2; four:
+ * 2048x2048 7.9 / 11.4, 4096x4864 28.3 / 24.2, 2048x896 8.0 / 7.0, Q5 1024x1536 9.8 / 9.2, 2048x2048 10.0 / 11.4. */
 bool few_wanted(bool q5, uint32_t nb, uint32_t ntok, uint64_t rows) {
     const uint32_t passes = (ntok + FEW_NT - 1) / FEW_NT;
     if (passes > 4 || 16 * passes > nb + 4 || (nb < 16 && rows * passes > 2048)) return false;
