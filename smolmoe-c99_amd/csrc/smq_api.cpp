@@ -50,9 +50,11 @@ thread_local bool t_capturing = false;
 
 /* Score workspaces of captured decode attention, each owned by one graph: a graph may be replayed on any stream,
  * beside eager work and other graphs. ready_ws waits for the open capture (used: it recorded a launch that writes
- * it); a graph that recorded one takes it along until smq_graph_destroy. */
+ * it); a graph that recorded one takes it along until smq_graph_destroy. One capture is open at a time, on the
+ * library's stream: a second begin must not touch what the first has recorded. */
 struct GraphScores {
     std::mutex mu;
+    bool open = false;
     float *ready_ws = nullptr;
     bool used = false;
     std::map<void *, float *> of_graph;
@@ -315,7 +317,9 @@ void smq_shutdown(void) {
         g_graph_scores.release();
         (void)hipFree(g_graph_scores.ready_ws);
         g_graph_scores.ready_ws = nullptr;
+        g_graph_scores.used = g_graph_scores.open = false;
     }
+    t_capturing = false;
     (void)hipFree(g.mq_ws);
     (void)hipStreamDestroy(g.own);
     g = Context();
@@ -1359,6 +1363,8 @@ smq_status smq_capture_begin(void) {
     if (g.cur != g.own) return set_status(SMQ_ERR_STATE, "capture needs the library stream");
     {
         std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        if (g_graph_scores.open) return set_status(SMQ_ERR_STATE, "a capture is open");
+        g_graph_scores.open = true;
         g_graph_scores.used = false;
         g_graph_scores.release();
         /* without it (no memory) the capture records the kernel that needs none */
@@ -1370,28 +1376,40 @@ smq_status smq_capture_begin(void) {
     }
     /* thread-local mode: a call from this thread that may not be captured (a synchronizing copy, an
      * allocation) fails the capture instead of being recorded or run behind the graph's back */
-    if (!hip_ok(hipStreamBeginCapture(g.cur, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
+    if (!hip_ok(hipStreamBeginCapture(g.cur, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture")) {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        g_graph_scores.open = false;
         return t_status;
+    }
     t_capturing = true;
     return SMQ_OK;
 }
 
 void *smq_capture_end(void) {
     if (!ready()) return nullptr;
+    const bool mine = t_capturing; /* else the program's own capture of the library's stream */
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    t_capturing = false;
-    if (!hip_ok(hipStreamEndCapture(g.cur, &graph), "hipStreamEndCapture")) return nullptr;
-    const bool ok = hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
-    (void)hipGraphDestroy(graph);
-    if (!ok) return nullptr;
-    std::lock_guard<std::mutex> l(g_graph_scores.mu);
-    if (g_graph_scores.used) {
-        g_graph_scores.of_graph[(void *)exec] = g_graph_scores.ready_ws;
-        g_graph_scores.ready_ws = nullptr;
-        g_graph_scores.used = false;
+    bool ok = hip_ok(hipStreamEndCapture(g.cur, &graph), "hipStreamEndCapture");
+    if (mine) {
+        /* a failed end closes the capture too, unless the stream was another one */
+        hipStreamCaptureStatus left = hipStreamCaptureStatusNone;
+        if (!ok && hipStreamIsCapturing(g.own, &left) == hipSuccess && left != hipStreamCaptureStatusNone) return nullptr;
+        t_capturing = false;
     }
-    return (void *)exec;
+    if (ok) {
+        ok = hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
+        (void)hipGraphDestroy(graph);
+    }
+    if (mine) {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        if (ok && g_graph_scores.used) {
+            g_graph_scores.of_graph[(void *)exec] = g_graph_scores.ready_ws;
+            g_graph_scores.ready_ws = nullptr;
+        }
+        g_graph_scores.used = g_graph_scores.open = false;
+    }
+    return ok ? (void *)exec : nullptr;
 }
 
 smq_status smq_graph_launch(void *graph) {

@@ -1,0 +1,162 @@
+"""Cases of tests/test_host.py, each in a process of its own: host_cases.py FAKE_HIP_LIBRARY CASE. The library's host code
+runs on the recording runtime of tests/fake_hip.cpp; nothing here needs a GPU."""
+import ctypes
+import os
+import sys
+import threading
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+fake = smq = None
+vp = ctypes.c_void_p
+
+
+class Shape(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_uint32) for n in ("heads", "kv_heads", "head_dim", "rotary_pairs", "window", "context")]
+
+
+def load(path):
+    global fake, smq
+    fake = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+    smq = ctypes.CDLL(os.path.join(ROOT, "smolmoe-c99_amd", "libsmq_gfx950.so"))
+    for lib, names in ((fake, ("fake_log", "fake_errors")), (smq, ("smq_last_error",))):
+        for n in names:
+            getattr(lib, n).restype = ctypes.c_char_p
+    for n in ("smq_malloc", "smq_capture_end", "smq_stream"):
+        getattr(smq, n).restype = vp
+    smq.smq_malloc.argtypes = [ctypes.c_size_t]
+    smq.smq_set_stream.argtypes = smq.smq_graph_launch.argtypes = smq.smq_graph_destroy.argtypes = [vp]
+    smq.smq_free.argtypes = [vp]
+    fake.fake_fail_size.argtypes = [ctypes.c_size_t]
+    fake.fake_allocations.restype = fake.fake_frees.restype = ctypes.c_uint64
+    u32 = ctypes.c_uint32
+    smq.smq_attention.argtypes = [vp, vp, vp, vp, u32, vp, u32, vp]
+    smq.smq_attention_rope_q8.argtypes = [vp] * 3 + [vp] + [vp] * 5 + [u32] + [vp] * 3
+    smq.smq_quantize_q5_rows.argtypes = [vp, u32, u32, vp]
+    smq.smq_matmul.argtypes = [vp, u32, vp, vp, u32]
+
+
+def init():
+    assert smq.smq_init(0) == 0, smq.smq_last_error()
+
+
+def log():
+    return [line.split() for line in fake.fake_log().decode().splitlines()]
+
+
+def kernels():
+    return [w[0] for w in log()]
+
+
+def errors():
+    return fake.fake_errors().decode()
+
+
+def stream():
+    s = vp()
+    assert fake.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    return s.value
+
+
+def on_thread(f):
+    out = []
+    t = threading.Thread(target=lambda: out.append(f()))
+    t.start()
+    t.join()
+    return out[0]
+
+
+class Attention:
+    """One token's attention (ntok: up to 256) with buffers of its own."""
+
+    def __init__(self, hd, heads=4, kv=2, context=2048, window=0):
+        self.shape = Shape(heads, kv, hd, hd // 2, window, context)
+        self.heads, self.hd, self.kvd, self.context = heads, hd, kv * hd, context
+        self.cache = [smq.smq_malloc(context * self.kvd * 4) for _ in range(2)]
+        self.pos = smq.smq_malloc(4)
+        self.rows = [smq.smq_malloc(256 * heads * hd * 4) for _ in range(2)]
+
+    def __call__(self, pos=1000, ntok=1, pos_dev=False):
+        q, att = self.rows
+        return smq.smq_attention(q, *self.cache, att, ntok, ctypes.byref(self.shape), pos, self.pos if pos_dev else None)
+
+
+class RopeAttention(Attention):
+    def __init__(self, hd, **kw):
+        super().__init__(hd, **kw)
+        n = self.heads * hd
+        self.b = [smq.smq_malloc(n * 4), smq.smq_malloc(self.kvd * 4), smq.smq_malloc(self.kvd * 4)]
+        self.tables = [smq.smq_malloc(self.context * hd * 2) for _ in range(2)]
+        self.out = [smq.smq_malloc(n * 4), smq.smq_malloc(n // 32 * 4), smq.smq_malloc(n)]
+
+    def __call__(self, pos=1000, pos_dev=False):
+        return smq.smq_attention_rope_q8(*self.b, ctypes.byref(self.shape), *self.tables, *self.cache, self.out[0], pos,
+                                         self.pos if pos_dev else None, self.out[1], self.out[2])
+
+
+def capture(f):
+    assert smq.smq_capture_begin() == 0, smq.smq_last_error()
+    assert f() == 0, smq.smq_last_error()
+    g = smq.smq_capture_end()
+    assert g, smq.smq_last_error()
+    return g
+
+
+def both_at_once(graphs, side):
+    """The graphs on two streams without an order between them."""
+    assert smq.smq_graph_launch(graphs[0]) == 0
+    smq.smq_set_stream(side)
+    assert smq.smq_graph_launch(graphs[1]) == 0
+    smq.smq_set_stream(None)
+
+
+def nested_capture():
+    """A begin inside an open capture, of the same thread or another, is refused and changes nothing: the graph still
+    owns the workspace that it recorded."""
+    for other in (False, True):
+        init()
+        att = Attention(128)
+        assert smq.smq_capture_begin() == 0
+        assert att() == 0
+        assert (on_thread(smq.smq_capture_begin) if other else smq.smq_capture_begin()) != 0
+        assert fake.hipGetLastError() == 0  # nothing for the next launch to find
+        first = smq.smq_capture_end()
+        assert first
+        second = capture(att)
+        fake.fake_clear()
+        both_at_once((first, second), stream())
+        assert len({w[8] for w in log()}) == 2, fake.fake_log().decode()
+        smq.smq_graph_destroy(second)
+        assert smq.smq_graph_launch(first) == 0
+        assert errors() == "", errors()
+        smq.smq_graph_destroy(first)
+        smq.smq_shutdown()
+
+
+def failed_captures():
+    """A capture that fails (a call that it does not allow) or is ended on the wrong stream leaves the next ones whole."""
+    init()
+    att, side = Attention(128), stream()
+    assert smq.smq_capture_begin() == 0 and att() == 0
+    assert smq.smq_malloc(64) is None
+    assert smq.smq_capture_end() is None
+    fake.hipGetLastError()
+    assert smq.smq_capture_begin() == 0 and att() == 0
+    smq.smq_set_stream(side)
+    assert smq.smq_capture_end() is None  # the library's stream is still capturing
+    fake.hipGetLastError()
+    smq.smq_set_stream(None)
+    assert smq.smq_capture_begin() != 0
+    first = smq.smq_capture_end()
+    assert first
+    second = capture(att)
+    fake.fake_clear()
+    both_at_once((first, second), side)
+    assert errors() == "", errors()
+
+
+CASES = [f for f in (nested_capture, failed_captures)]
+
+if __name__ == "__main__":
+    load(sys.argv[1])
+    {f.__name__: f for f in CASES}[sys.argv[2]]()
+    print("ok")
