@@ -1420,13 +1420,17 @@ smq_status smq_graph_launch(void *graph) {
 
 void smq_graph_destroy(void *graph) {
     if (!graph) return;
+    {
+        /* before the handle is free: another thread's capture may get the same one at once */
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        auto it = g_graph_scores.of_graph.find(graph);
+        if (it != g_graph_scores.of_graph.end()) {
+            g_graph_scores.retired.push_back(it->second);
+            g_graph_scores.of_graph.erase(it);
+        }
+    }
     (void)hipGraphExecDestroy((hipGraphExec_t)graph);
     std::lock_guard<std::mutex> l(g_graph_scores.mu);
-    auto it = g_graph_scores.of_graph.find(graph);
-    if (it != g_graph_scores.of_graph.end()) {
-        g_graph_scores.retired.push_back(it->second);
-        g_graph_scores.of_graph.erase(it);
-    }
     if (!t_capturing) g_graph_scores.release();
 }
 

@@ -154,7 +154,21 @@ def failed_captures():
     assert errors() == "", errors()
 
 
-CASES = [f for f in (nested_capture, failed_captures)]
+def destroyed_handle():
+    """A graph made while another is destroyed may get its handle, and keeps its own workspace."""
+    init()
+    att, made = Attention(128), []
+    first = capture(att)
+    hook = ctypes.CFUNCTYPE(None)(lambda: made.append(capture(att)))
+    fake.fake_on_exec_destroy(hook)
+    smq.smq_graph_destroy(first)
+    assert made == [first]  # the handle again
+    capture(att)
+    assert smq.smq_graph_launch(made[0]) == 0
+    assert errors() == "", errors()
+
+
+CASES = [f for f in (nested_capture, failed_captures, destroyed_handle)]
 
 if __name__ == "__main__":
     load(sys.argv[1])
