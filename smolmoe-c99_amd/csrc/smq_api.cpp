@@ -1026,8 +1026,8 @@ smq_status smq_rope_kv(float *q, float *k, const float *v, uint32_t ntok, const 
 /* Attention of checked operands. The score workspace of the prefill kernels and of decode at head sizes other than
  * 64 belongs to the library's own stream, or in smq_capture_begin's captures to the graph: work on another stream
  * or in a capture that the library did not open takes the kernels that need none. One thread at a time enqueues
- * the launches that share it. */
-static smq_status attention_launch(const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
+ * the launches that share it. s: the stream of the whole call, read once (smq_set_stream on another thread). */
+static smq_status attention_launch(hipStream_t s, const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
                                    const smq::AttnShape &sh, uint32_t pos0, const int32_t *pos_dev, float *xd,
                                    int8_t *xq, const char *who) {
     static std::mutex mu;
@@ -1035,7 +1035,7 @@ static smq_status attention_launch(const float *q, const float *keys, const floa
     float *ws = nullptr, *scores = g.scores;
     const bool decode_ws = ntok == 1 && smq::attention_decode_split(sh, q, keys, values, pos0, pos_dev);
     if (decode_ws) scores = nullptr;
-    if ((ntok > 1 || decode_ws) && g.cur == g.own) {
+    if ((ntok > 1 || decode_ws) && s == g.own) {
         if (t_capturing) {
             if (decode_ws) {
                 std::lock_guard<std::mutex> l(g_graph_scores.mu);
@@ -1044,14 +1044,14 @@ static smq_status attention_launch(const float *q, const float *keys, const floa
             }
         } else {
             hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
-            if (!hip_ok(hipStreamIsCapturing(g.cur, &capture), who)) return t_status;
+            if (!hip_ok(hipStreamIsCapturing(s, &capture), who)) return t_status;
             if (capture == hipStreamCaptureStatusNone) {
                 (decode_ws ? scores : ws) = g.tiles_ws;
                 lock.lock();
             }
         }
     }
-    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, g.cur, scores, ws,
+    return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, s, scores, ws,
                                         ws ? smq::TILES_WORKSPACE_BYTES : 0),
                   who)
                ? SMQ_OK
@@ -1071,7 +1071,7 @@ smq_status smq_attention(const float *q, const float *keys, const float *values,
         !extent_ok(keys, cache, "keys") || !extent_ok(values, cache, "values") ||
         !extent_ok(pos_dev, pos_dev ? 4 : 0, "pos"))
         return t_status;
-    return attention_launch(q, keys, values, att, ntok, sh, pos0, pos_dev, nullptr, nullptr, "attention");
+    return attention_launch(g.cur, q, keys, values, att, ntok, sh, pos0, pos_dev, nullptr, nullptr, "attention");
 }
 
 smq_status smq_attention_q8(const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
@@ -1089,11 +1089,12 @@ smq_status smq_attention_q8(const float *q, const float *keys, const float *valu
         !extent_ok(pos_dev, pos_dev ? 4 : 0, "pos") || !extent_ok(xd, ntok * nbq * 4, "xd") ||
         !extent_ok(xq, ntok * nbq * smq::QK, "xq"))
         return t_status;
+    const hipStream_t s = g.cur;
     if (sh.head_dim % smq::QK == 0) /* each head owns whole blocks: quantized in the same kernel */
-        return attention_launch(q, keys, values, att, ntok, sh, pos0, pos_dev, xd, xq, "attention_q8");
-    if (attention_launch(q, keys, values, att, ntok, sh, pos0, pos_dev, nullptr, nullptr, "attention_q8") != SMQ_OK)
+        return attention_launch(s, q, keys, values, att, ntok, sh, pos0, pos_dev, xd, xq, "attention_q8");
+    if (attention_launch(s, q, keys, values, att, ntok, sh, pos0, pos_dev, nullptr, nullptr, "attention_q8") != SMQ_OK)
         return t_status;
-    return hip_ok(smq::launch_quantize_q8(att, ntok, sh.q_dim, xd, xq, g.flag, g.cur), "attention_q8") ? SMQ_OK
+    return hip_ok(smq::launch_quantize_q8(att, ntok, sh.q_dim, xd, xq, g.flag, s), "attention_q8") ? SMQ_OK
                                                                                                         : t_status;
 }
 

@@ -49,7 +49,7 @@ std::string log_text, error_text;
 uintptr_t next_address = 0x100000000000ull, next_handle = 0x1000;
 size_t fail_size = 0;
 uint64_t allocations = 0, frees = 0;
-void (*on_exec_destroy)() = nullptr;
+void (*on_exec_destroy)() = nullptr, (*on_is_capturing)() = nullptr; /* called once: what another thread may do there */
 hipError_t last = hipSuccess;
 struct Config {
     dim3 grid, block;
@@ -66,6 +66,11 @@ void error(const std::string &s) { error_text += s + "\n"; }
 void merge(Clock &a, const Clock &b) {
     for (auto &x : b)
         if (a[x.first] < x.second) a[x.first] = x.second;
+}
+void once(void (*&hook)()) {
+    void (*f)() = hook;
+    hook = nullptr;
+    if (f) f();
 }
 bool forbidden() { /* inside a capture of this thread */
     for (auto &s : streams)
@@ -116,6 +121,7 @@ void fake_fail_size(size_t n) { fail_size = n; }
 uint64_t fake_allocations() { return allocations; }
 uint64_t fake_frees() { return frees; }
 void fake_on_exec_destroy(void (*f)()) { on_exec_destroy = f; }
+void fake_on_is_capturing(void (*f)()) { on_is_capturing = f; }
 
 void **__hipRegisterFatBinary(const void *) {
     static void *h[1];
@@ -244,6 +250,7 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
     *c = !streams[s].capturing ? hipStreamCaptureStatusNone
                                : streams[s].invalid ? hipStreamCaptureStatusInvalidated : hipStreamCaptureStatusActive;
+    once(on_is_capturing);
     return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
@@ -275,11 +282,7 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
     if (!execs.count(e)) return ret(hipErrorInvalidValue);
     execs[e].dead = true;
     free_execs.push_back(e);
-    if (on_exec_destroy) { /* what another thread may do once the handle is free */
-        void (*f)() = on_exec_destroy;
-        on_exec_destroy = nullptr;
-        f();
-    }
+    once(on_exec_destroy);
     return hipSuccess;
 }
 

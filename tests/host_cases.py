@@ -168,7 +168,21 @@ def destroyed_handle():
     assert errors() == "", errors()
 
 
-CASES = [f for f in (nested_capture, failed_captures, destroyed_handle)]
+def stream_read_once():
+    """A stream set by another thread during a call does not move the rest of the call, nor the workspace with it."""
+    init()
+    own, side = smq.smq_stream(), stream()
+    hook = ctypes.CFUNCTYPE(None)(lambda: smq.smq_set_stream(side))
+    for att, ntok in ((Attention(128), 1), (Attention(128), 200), (Attention(48), 200)):
+        smq.smq_set_stream(None)
+        fake.fake_clear()
+        fake.fake_on_is_capturing(hook)
+        assert att(ntok=ntok) == 0
+        assert smq.smq_stream() == side and log()
+        assert {int(w[6], 16) for w in log()} == {own}, fake.fake_log().decode()
+
+
+CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once)]
 
 if __name__ == "__main__":
     load(sys.argv[1])
