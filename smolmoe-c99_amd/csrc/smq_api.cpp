@@ -66,6 +66,19 @@ struct GraphScores {
 };
 GraphScores g_graph_scores;
 
+/* Who uses the library's own score workspaces. g.scores, for eager decode attention at head size 64, serves any stream:
+ * it passes to another one only when its last use is over (a synchronization of its user through the library) or,
+ * from the library's own stream, by an event; no other stream is known to exist still. mu is held while launches that
+ * share a workspace are enqueued. */
+struct SharedScores {
+    std::mutex mu;
+    hipStream_t user = nullptr;
+    bool busy = false;
+    uint64_t uses = 0;
+    hipEvent_t handed = nullptr;
+};
+SharedScores g_shared;
+
 /* The library's own allocations (smq_malloc), base -> size: extent checks look here first, so a
  * check needs no runtime call for them, and none at all runs inside a stream capture. */
 std::mutex g_alloc_mu;
@@ -106,6 +119,38 @@ bool ready() {
     if (g.ready) return true;
     set_status(SMQ_ERR_STATE, "smq_init has not been called");
     return false;
+}
+
+/* Waits for s, and for the workspace where s used it last. */
+hipError_t finish(hipStream_t s) {
+    uint64_t uses = 0;
+    {
+        std::lock_guard<std::mutex> l(g_shared.mu);
+        if (g_shared.user == s) uses = g_shared.uses;
+    }
+    const hipError_t e = hipStreamSynchronize(s);
+    std::lock_guard<std::mutex> l(g_shared.mu);
+    if (e == hipSuccess && g_shared.user == s && g_shared.uses == uses) g_shared.busy = false;
+    return e;
+}
+
+/* g.scores for s's next launches, or null. g_shared.mu is held. */
+float *take_scores(hipStream_t s) {
+    if (g_shared.busy && g_shared.user != s) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+        if (g_shared.user != g.own || hipStreamIsCapturing(g.own, &capture) != hipSuccess ||
+            capture != hipStreamCaptureStatusNone)
+            return nullptr;
+        if (hipEventRecord(g_shared.handed, g.own) != hipSuccess ||
+            hipStreamWaitEvent(s, g_shared.handed, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    g_shared.user = s;
+    g_shared.busy = true;
+    ++g_shared.uses;
+    return g.scores;
 }
 
 /* The byte range [p, p + bytes) must lie inside one device allocation. */
@@ -238,7 +283,7 @@ float dot_impl(bool q5, const unsigned char *w, const float *xd, const int8_t *x
     if (t_status != SMQ_OK) return 0.0f;
     float v = 0.0f;
     if (!hip_ok(hipMemcpyAsync(&v, g.scalar, sizeof(v), hipMemcpyDeviceToHost, g.cur), "dot") ||
-        !hip_ok(hipStreamSynchronize(g.cur), "dot"))
+        !hip_ok(finish(g.cur), "dot"))
         return 0.0f;
     return v;
 }
@@ -283,6 +328,7 @@ smq_status smq_init(int device) {
     if (!hip_ok(hipMalloc((void **)&g.scores, smq::SCORE_WORKSPACE_BYTES), "hipMalloc")) return t_status;
     if (!hip_ok(hipMalloc((void **)&g.mq_ws, smq::MQ_WORKSPACE_BYTES), "hipMalloc")) return t_status;
     if (!hip_ok(hipMalloc((void **)&g.tiles_ws, smq::TILES_WORKSPACE_BYTES), "hipMalloc")) return t_status;
+    if (!hip_ok(hipEventCreateWithFlags(&g_shared.handed, hipEventDisableTiming), "hipEventCreate")) return t_status;
     if (!hip_ok(hipEventCreate(&g.t0), "hipEventCreate") || !hip_ok(hipEventCreate(&g.t1), "hipEventCreate"))
         return t_status;
     /* the allocation-free argmax's static partials: their device address, once, with the device current */
@@ -308,6 +354,9 @@ void smq_shutdown(void) {
     (void)hipStreamSynchronize(g.cur);
     (void)hipEventDestroy(g.t0);
     (void)hipEventDestroy(g.t1);
+    (void)hipEventDestroy(g_shared.handed);
+    g_shared.user = nullptr;
+    g_shared.busy = false;
     (void)hipFree(g.flag);
     (void)hipFree(g.argmax_parts);
     (void)hipFree(g.scores);
@@ -335,7 +384,7 @@ smq_status smq_set_stream(void *s) {
 
 smq_status smq_synchronize(void) {
     if (!ready()) return t_status;
-    return hip_ok(hipStreamSynchronize(g.cur), "hipStreamSynchronize") ? SMQ_OK : t_status;
+    return hip_ok(finish(g.cur), "hipStreamSynchronize") ? SMQ_OK : t_status;
 }
 
 const char *smq_device_arch(void) { return g.ready ? g.arch : ""; }
@@ -369,7 +418,7 @@ int smq_quantize_q8(const float *x, uint32_t n, float *d, int8_t *q) {
     if (!hip_ok(hipMemsetAsync(g.qflag, 0, sizeof(int), g.cur), "quantize_q8") ||
         !hip_ok(smq::launch_quantize_q8(x, 1, n, d, q, g.qflag, g.cur), "quantize_q8") ||
         !hip_ok(hipMemcpyAsync(&bad, g.qflag, sizeof(int), hipMemcpyDeviceToHost, g.cur), "quantize_q8") ||
-        !hip_ok(hipStreamSynchronize(g.cur), "quantize_q8"))
+        !hip_ok(finish(g.cur), "quantize_q8"))
         return -1;
     return bad ? -1 : 0;
 }
@@ -968,7 +1017,7 @@ smq_status smq_matmul_glu(const smq_qmat *gate, const smq_qmat *up, const smq_ac
 smq_status smq_numeric_check(void) {
     if (!ready()) return t_status;
     int bad = 0;
-    if (!hip_ok(hipStreamSynchronize(g.cur), "numeric_check") ||
+    if (!hip_ok(finish(g.cur), "numeric_check") ||
         !hip_ok(hipMemcpy(&bad, g.flag, sizeof(int), hipMemcpyDeviceToHost), "numeric_check"))
         return t_status;
     if (!bad) return SMQ_OK;
@@ -1023,32 +1072,44 @@ smq_status smq_rope_kv(float *q, float *k, const float *v, uint32_t ntok, const 
                : t_status;
 }
 
-/* Attention of checked operands. The score workspace of the prefill kernels and of decode at head sizes other than
- * 64 belongs to the library's own stream, or in smq_capture_begin's captures to the graph: work on another stream
- * or in a capture that the library did not open takes the kernels that need none. One thread at a time enqueues
- * the launches that share it. s: the stream of the whole call, read once (smq_set_stream on another thread). */
+/* The score workspace of one token's attention on s: the graph's in smq_capture_begin's captures, the library's outside
+ * captures (split, head sizes other than 64: on its own stream; lock is taken), else none. False: an error is set. */
+static bool decode_scores(hipStream_t s, bool split, float **scores, std::unique_lock<std::mutex> &lock, const char *who) {
+    *scores = nullptr;
+    if (t_capturing && s == g.own) {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        *scores = g_graph_scores.ready_ws;
+        g_graph_scores.used = *scores != nullptr;
+        return true;
+    }
+    if (split && s != g.own) return true;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+    if (!hip_ok(hipStreamIsCapturing(s, &capture), who)) return false;
+    if (capture == hipStreamCaptureStatusNone) {
+        lock.lock();
+        *scores = split ? g.tiles_ws : take_scores(s);
+    }
+    return true;
+}
+
+/* Attention of checked operands. The score workspace of the prefill kernels belongs to the library's own stream: work
+ * on another stream or in a capture takes the kernels that need none. One thread at a time enqueues the launches that
+ * share a workspace. s: the stream of the whole call, read once (smq_set_stream on another thread). */
 static smq_status attention_launch(hipStream_t s, const float *q, const float *keys, const float *values, float *att, uint32_t ntok,
                                    const smq::AttnShape &sh, uint32_t pos0, const int32_t *pos_dev, float *xd,
                                    int8_t *xq, const char *who) {
-    static std::mutex mu;
-    std::unique_lock<std::mutex> lock(mu, std::defer_lock);
-    float *ws = nullptr, *scores = g.scores;
-    const bool decode_ws = ntok == 1 && smq::attention_decode_split(sh, q, keys, values, pos0, pos_dev);
-    if (decode_ws) scores = nullptr;
-    if ((ntok > 1 || decode_ws) && s == g.own) {
-        if (t_capturing) {
-            if (decode_ws) {
-                std::lock_guard<std::mutex> l(g_graph_scores.mu);
-                scores = g_graph_scores.ready_ws;
-                g_graph_scores.used = scores != nullptr;
-            }
-        } else {
-            hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
-            if (!hip_ok(hipStreamIsCapturing(s, &capture), who)) return t_status;
-            if (capture == hipStreamCaptureStatusNone) {
-                (decode_ws ? scores : ws) = g.tiles_ws;
-                lock.lock();
-            }
+    std::unique_lock<std::mutex> lock(g_shared.mu, std::defer_lock);
+    float *ws = nullptr, *scores = nullptr;
+    if (ntok == 1) {
+        const bool split = smq::attention_decode_split(sh, q, keys, values, pos0, pos_dev);
+        if ((split || smq::attention_decode_rows(sh, q, keys, values)) && !decode_scores(s, split, &scores, lock, who))
+            return t_status;
+    } else if (s == g.own && !t_capturing) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+        if (!hip_ok(hipStreamIsCapturing(s, &capture), who)) return t_status;
+        if (capture == hipStreamCaptureStatusNone) {
+            ws = g.tiles_ws;
+            lock.lock();
         }
     }
     return hip_ok(smq::launch_attention(q, keys, values, att, ntok, sh, pos0, pos_dev, g.flag, xd, xq, s, scores, ws,
@@ -1115,12 +1176,18 @@ smq_status smq_attention_rope_q8(float *q, float *k, const float *v, const smq_a
         !extent_ok(xq, nbq * smq::QK, "xq"))
         return t_status;
     const bool aligned = !((uintptr_t)q & 15) && !((uintptr_t)k & 15) && !((uintptr_t)v & 15);
-    if (aligned && smq::attention_rows_ok(sh, q, keys, values))
+    if (aligned && smq::attention_rows_ok(sh, q, keys, values)) {
+        const hipStream_t s = g.cur;
+        std::unique_lock<std::mutex> lock(g_shared.mu, std::defer_lock);
+        float *scores = nullptr;
+        if (smq::attention_decode_rows(sh, q, keys, values) && !decode_scores(s, false, &scores, lock, "attention_rope_q8"))
+            return t_status;
         return hip_ok(smq::launch_attention_rope(q, k, v, cos_table, sin_table, keys, values, att, sh, pos0, pos_dev,
-                                                 g.flag, xd, xq, g.scores, g.cur),
+                                                 g.flag, xd, xq, scores, s),
                       "attention_rope_q8")
                    ? SMQ_OK
                    : t_status;
+    }
     /* other shapes: the two-step form (q and k are left rotated) */
     if (smq_rope_kv(q, k, v, 1, shape, cos_table, sin_table, keys, values, pos0, pos_dev) != SMQ_OK) return t_status;
     return smq_attention_q8(q, keys, values, att, 1, shape, pos0, pos_dev, xd, xq);
@@ -1330,7 +1397,7 @@ smq_status smq_memcpy_htod(void *dst, const void *src, size_t bytes) {
     if (!bytes) return SMQ_OK;
     if (!extent_ok(dst, bytes, "dst")) return t_status;
     if (!hip_ok(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g.cur), "memcpy htod") ||
-        !hip_ok(hipStreamSynchronize(g.cur), "memcpy htod"))
+        !hip_ok(finish(g.cur), "memcpy htod"))
         return t_status;
     return SMQ_OK;
 }
@@ -1340,7 +1407,7 @@ smq_status smq_memcpy_dtoh(void *dst, const void *src, size_t bytes) {
     if (!bytes) return SMQ_OK;
     if (!extent_ok(src, bytes, "src")) return t_status;
     if (!hip_ok(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g.cur), "memcpy dtoh") ||
-        !hip_ok(hipStreamSynchronize(g.cur), "memcpy dtoh"))
+        !hip_ok(finish(g.cur), "memcpy dtoh"))
         return t_status;
     return SMQ_OK;
 }

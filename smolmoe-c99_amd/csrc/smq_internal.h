@@ -199,8 +199,9 @@ struct AttnShape {
 hipError_t launch_rope_kv(float *q, float *k, const float *v, uint32_t ntok, const AttnShape &sh, const float *cs,
                           const float *sn, float *kcache, float *vcache, uint32_t pos0, const int32_t *pos_dev,
                           int *flag, hipStream_t s);
-/* Whether one token's attention at a head size other than 64 takes the two launches that need `scores`
- * (SCORE_WORKSPACE_BYTES, not shared with a call that may overlap); without them one launch, no workspace. */
+/* Whether one token's attention takes the two launches that need `scores` (SCORE_WORKSPACE_BYTES, not shared with a call
+ * that may overlap), at head size 64 and at other multiples of 32; without them one launch, no workspace. */
+bool attention_decode_rows(const AttnShape &sh, const void *q, const void *kcache, const void *vcache);
 bool attention_decode_split(const AttnShape &sh, const void *q, const void *kcache, const void *vcache, uint32_t pos0,
                             bool pos_dev);
 hipError_t launch_attention(const float *q, const float *kcache, const float *vcache, float *att, uint32_t ntok,

@@ -3077,6 +3077,11 @@ bool attention_rows_ok(const AttnShape &sh, const void *q, const void *kcache, c
            ((uintptr_t)vcache & 15) == 0;
 }
 
+bool attention_decode_rows(const AttnShape &sh, const void *q, const void *kcache, const void *vcache) {
+    return attention_rows_ok(sh, q, kcache, vcache) && (size_t)sh.heads * sh.context <= MAX_SCORE_FLOATS &&
+           sh.heads / sh.kv_heads <= AS_MAXG;
+}
+
 /* One token at head sizes other than 64 in two launches, from the position where they beat k_attend's one workgroup
  * per head and 32 columns. Measured on MI355X, us, two launches / one: 12 heads of 128 at 41 positions 8.7 / 7.1, 101
  * 8.8 / 8.3, 201 8.8 / 10.3, 401 10.4 / 14.9, 3072 26 / 83; 9 heads of 32 at 201 8.6 / 7.9, 301 9.1 / 10.3; 4 heads
@@ -3131,8 +3136,7 @@ hipError_t launch_attention(const float *q, const float *kcache, const float *vc
         attend_tiles_ok(sh, q, kcache, vcache, ntok, pos0, tiles_ws_bytes))
         return launch_attend_tiles(q, kcache, vcache, att, ntok, sh, pos0, flag, xd, xq, tiles_ws, tiles_ws_bytes, s);
     const uint32_t groups = (sh.head_dim + ATT_JW - 1) / ATT_JW;
-    if (ntok == 1 && scores && attention_rows_ok(sh, q, kcache, vcache) &&
-        (size_t)sh.heads * sh.context <= MAX_SCORE_FLOATS && sh.heads / sh.kv_heads <= AS_MAXG) {
+    if (ntok == 1 && scores && attention_decode_rows(sh, q, kcache, vcache)) {
         /* one decoding token whose q is rotated and whose k and v rows are in the caches already:
          * the scores spread over workgroups of positions, then the values */
         const size_t lds = (((size_t)sh.context + 3) / 4 * 4 + (size_t)AR_FIXED) * sizeof(float);
@@ -3202,7 +3206,7 @@ hipError_t launch_attention_rope(const float *q, const float *k, const float *v,
     const uint32_t groups = (sh.head_dim + ATT_JW - 1) / ATT_JW;
     const size_t lds = (((size_t)sh.context + 3) / 4 * 4 + (size_t)AR_FIXED) * sizeof(float);
     RopeRows rr = {k, v, cs, sn};
-    if (scores && (size_t)sh.heads * sh.context <= MAX_SCORE_FLOATS && sh.heads / sh.kv_heads <= AS_MAXG) {
+    if (scores && attention_decode_rows(sh, q, kcache, vcache)) {
         const dim3 sgrid((sh.context + AS_SP - 1) / AS_SP, sh.kv_heads);
         hipLaunchKernelGGL(k_attend_scores<true>, sgrid, dim3(AS_WG), 0, s, q, kcache, vcache, sh, pos0, pos_dev, flag,
                            rr, scores);

@@ -182,7 +182,57 @@ def stream_read_once():
         assert {int(w[6], 16) for w in log()} == {own}, fake.fake_log().decode()
 
 
-CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once)]
+def two_launches():
+    names = kernels()
+    return any("k_attend_scores" in n for n in names) and any("k_attend_values" in n for n in names)
+
+
+def scores_by_stream():
+    """Decode attention in graphs, beside eager calls and on other streams: no two uses of a workspace without an order,
+    and two launches wherever the workspace can be had."""
+    for make in (lambda: Attention(64), lambda: RopeAttention(64), lambda: Attention(128)):
+        init()
+        att, own, side, third = make(), smq.smq_stream(), stream(), stream()
+        split = att.hd != 64  # on the library's own stream only
+        graphs = [capture(lambda: att(pos_dev=True)) for _ in range(2)]
+        fake.fake_clear()
+        both_at_once(graphs, side)
+        assert att() == 0  # eager, beside both
+        assert two_launches() and errors() == "", errors()
+
+        def call(s, expected):
+            fake.fake_clear()
+            smq.smq_set_stream(s)
+            assert att() == 0
+            assert two_launches() == expected and errors() == "", fake.fake_log().decode() + errors()
+
+        call(side, not split)  # from the library's stream to another: in order by an event
+        call(None, split)  # the other stream's use may be running: the launch that needs no workspace
+        call(third, False)
+        call(side, not split)
+        assert smq.smq_synchronize() == 0
+        for s in (third, side, None):  # after a synchronization of its user every stream may have it
+            call(s, not split or s is None)
+            assert smq.smq_synchronize() == 0
+
+        for s in (side, own):  # a capture that the program opened itself
+            smq.smq_set_stream(s)
+            assert fake.hipStreamBeginCapture(vp(s), 1) == 0
+            assert att() == 0
+            graph, exe = vp(), vp()
+            assert fake.hipStreamEndCapture(vp(s), ctypes.byref(graph)) == 0
+            assert fake.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+            smq.smq_set_stream(None)
+            assert att() == 0
+            fake.fake_clear()
+            assert fake.hipGraphLaunch(exe, vp(third)) == 0
+            assert not two_launches() and errors() == "", errors()
+        for g in graphs:
+            smq.smq_graph_destroy(g)
+        smq.smq_shutdown()
+
+
+CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream)]
 
 if __name__ == "__main__":
     load(sys.argv[1])

@@ -79,9 +79,10 @@ def test_attend_decode(orc, heads, kv_heads, hd, window, context, positions):
     graph.destroy()
 
 
-def test_graphs_own_their_scores(orc):
+@pytest.mark.parametrize("heads,kv_heads,hd", [(12, 2, 128), (14, 2, 64)])
+def test_graphs_own_their_scores(orc, heads, kv_heads, hd):
     """Two graphs of attention on two streams at once, replayed many times beside eager calls."""
-    heads, kv_heads, hd, context, pos = 12, 2, 128, 1024, 1000
+    context, pos = 1024, 1000
     qd, kd = heads * hd, kv_heads * hd
     shape = smq.attn_shape(heads, kv_heads, hd, hd // 2, 0, context)
     sets = []
