@@ -32,7 +32,7 @@ struct Context {
     float *scalar = nullptr;
     void *argmax_parts = nullptr; /* smq::MAX_ARGMAX_PARTS partials of the two-stage argmax */
     float *scores = nullptr;      /* decode attention scores (heads x context), smq::SCORE_WORKSPACE_BYTES */
-    float *tiles_ws = nullptr;    /* prefill attention scores, smq::TILES_WORKSPACE_BYTES */
+    float *tiles_ws = nullptr;    /* prefill attention scores, smq::TILES_WORKSPACE_BYTES, or null */
     float *mq_ws = nullptr;       /* split-K partial sums of the MFMA prefill GEMM, smq::MQ_WORKSPACE_BYTES */
     hipEvent_t t0 = nullptr, t1 = nullptr;
     int fast = 0;
@@ -327,7 +327,11 @@ smq_status smq_init(int device) {
         return t_status;
     if (!hip_ok(hipMalloc((void **)&g.scores, smq::SCORE_WORKSPACE_BYTES), "hipMalloc")) return t_status;
     if (!hip_ok(hipMalloc((void **)&g.mq_ws, smq::MQ_WORKSPACE_BYTES), "hipMalloc")) return t_status;
-    if (!hip_ok(hipMalloc((void **)&g.tiles_ws, smq::TILES_WORKSPACE_BYTES), "hipMalloc")) return t_status;
+    /* without it (no memory) attention takes the kernels that need none */
+    if (hipMalloc((void **)&g.tiles_ws, smq::TILES_WORKSPACE_BYTES) != hipSuccess) {
+        g.tiles_ws = nullptr;
+        (void)hipGetLastError();
+    }
     if (!hip_ok(hipEventCreateWithFlags(&g_shared.handed, hipEventDisableTiming), "hipEventCreate")) return t_status;
     if (!hip_ok(hipEventCreate(&g.t0), "hipEventCreate") || !hip_ok(hipEventCreate(&g.t1), "hipEventCreate"))
         return t_status;

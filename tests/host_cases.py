@@ -232,7 +232,25 @@ def scores_by_stream():
         smq.smq_shutdown()
 
 
-CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream)]
+def no_memory():
+    """Without memory for a score workspace the library starts, captures and computes with the kernels that need none."""
+    fake.fake_fail_size(128 << 20)
+    init()
+    for hd, ntok in ((128, 1), (64, 1), (128, 200), (64, 200)):
+        att = Attention(hd)
+        fake.fake_clear()
+        assert att(ntok=ntok) == 0, smq.smq_last_error()
+        assert log() and not any("k_ap_" in n for n in kernels()) and errors() == ""
+    fake.fake_fail_size(16 << 20)
+    graphs = [capture(Attention(hd)) for hd in (128, 64, 128, 64)]
+    for g in graphs:
+        fake.fake_clear()
+        assert smq.smq_graph_launch(g) == 0
+        assert log() and errors() == "", errors()
+        smq.smq_graph_destroy(g)
+
+
+CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream, no_memory)]
 
 if __name__ == "__main__":
     load(sys.argv[1])
