@@ -49,19 +49,79 @@ thread_local char t_message[1024];
 thread_local bool t_capturing = false;
 
 /* Score workspaces of captured decode attention, each owned by one graph: a graph may be replayed on any stream,
- * beside eager work and other graphs. ready_ws waits for the open capture (used: it recorded a launch that writes
- * it); a graph that recorded one takes it along until smq_graph_destroy. One capture is open at a time, on the
- * library's stream: a second begin must not touch what the first has recorded. */
+ * beside eager work and other graphs. `ready` waits for the open capture (used: it recorded a launch that writes it);
+ * a graph that recorded one takes it along until smq_graph_destroy. One capture is open at a time, on the library's
+ * stream: a second begin must not touch what the first has recorded. A destroyed graph's workspace is kept for a later
+ * capture, up to MAX_SPARE of them, and serves it once the replays are over (`done`, recorded on the library's
+ * stream): a program that captures again after each prompt allocates nothing and waits for nothing. */
 struct GraphScores {
+    static constexpr int MAX_SPARE = 4;
+    struct Item {
+        float *p;
+        hipEvent_t done;
+        void *exec;
+        bool elsewhere; /* replayed on a stream that `done` says nothing about: freed, which waits for the device */
+        Item *next;
+    };
     std::mutex mu;
-    bool open = false;
-    float *ready_ws = nullptr;
-    bool used = false;
-    std::map<void *, float *> of_graph;
-    std::vector<float *> retired; /* of graphs destroyed inside a capture, where nothing may be freed */
-    void release() {              /* not inside a capture; hipFree waits for a replay in flight */
-        for (float *p : retired) (void)hipFree(p);
-        retired.clear();
+    bool open = false, used = false;
+    Item *ready = nullptr, *owned = nullptr, *spare = nullptr;
+    Item *retired = nullptr; /* to be freed outside a capture */
+
+    static Item *make() { /* null where there is no memory: the capture records the kernel that needs none */
+        Item *i = new (std::nothrow) Item();
+        if (!i) return nullptr;
+        if (hipMalloc((void **)&i->p, smq::SCORE_WORKSPACE_BYTES) == hipSuccess) {
+            if (hipEventCreateWithFlags(&i->done, hipEventDisableTiming) == hipSuccess) return i;
+            (void)hipFree(i->p);
+        }
+        (void)hipGetLastError();
+        delete i;
+        return nullptr;
+    }
+    static void drop(Item *i) { /* not inside a capture; hipFree waits for a replay in flight */
+        if (!i) return;
+        (void)hipFree(i->p);
+        (void)hipEventDestroy(i->done);
+        delete i;
+    }
+    static void drop_all(Item *&list) {
+        while (list) {
+            Item *i = list;
+            list = i->next;
+            drop(i);
+        }
+    }
+    static void push(Item *&list, Item *i) {
+        i->next = list;
+        list = i;
+    }
+    Item *unlink(void *exec) {
+        for (Item **at = &owned; *at; at = &(*at)->next)
+            if ((*at)->exec == exec) {
+                Item *i = *at;
+                *at = i->next;
+                return i;
+            }
+        return nullptr;
+    }
+    /* a spare one whose replays are over, or a new one */
+    Item *take() {
+        for (Item **at = &spare; *at; at = &(*at)->next) {
+            if (hipEventQuery((*at)->done) != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
+            }
+            Item *i = *at;
+            *at = i->next;
+            return i;
+        }
+        return make();
+    }
+    int spares() const {
+        int n = 0;
+        for (Item *i = spare; i; i = i->next) ++n;
+        return n;
     }
 };
 GraphScores g_graph_scores;
@@ -341,6 +401,10 @@ smq_status smq_init(int device) {
         !hip_ok(smq::prepare_fused_attributes(), "hipFuncSetAttribute(fused GEMV)") ||
         !hip_ok(smq::prepare_mq8_attributes(), "hipFuncSetAttribute(MFMA GEMM)"))
         return t_status;
+    {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        if (!g_graph_scores.ready) g_graph_scores.ready = GraphScores::make();
+    }
     g.cur = g.own;
     g.device = device;
     const char *env = getenv("SMQ_CHECKS");
@@ -367,10 +431,12 @@ void smq_shutdown(void) {
     (void)hipFree(g.tiles_ws);
     {
         std::lock_guard<std::mutex> l(g_graph_scores.mu);
-        g_graph_scores.release();
-        (void)hipFree(g_graph_scores.ready_ws);
-        g_graph_scores.ready_ws = nullptr;
+        GraphScores::drop_all(g_graph_scores.retired);
+        GraphScores::drop_all(g_graph_scores.spare);
+        GraphScores::drop(g_graph_scores.ready);
+        g_graph_scores.ready = nullptr;
         g_graph_scores.used = g_graph_scores.open = false;
+        for (GraphScores::Item *i = g_graph_scores.owned; i; i = i->next) i->elsewhere = true; /* the stream goes */
     }
     t_capturing = false;
     (void)hipFree(g.mq_ws);
@@ -1082,7 +1148,7 @@ static bool decode_scores(hipStream_t s, bool split, float **scores, std::unique
     *scores = nullptr;
     if (t_capturing && s == g.own) {
         std::lock_guard<std::mutex> l(g_graph_scores.mu);
-        *scores = g_graph_scores.ready_ws;
+        *scores = g_graph_scores.ready ? g_graph_scores.ready->p : nullptr;
         g_graph_scores.used = *scores != nullptr;
         return true;
     }
@@ -1438,13 +1504,8 @@ smq_status smq_capture_begin(void) {
         if (g_graph_scores.open) return set_status(SMQ_ERR_STATE, "a capture is open");
         g_graph_scores.open = true;
         g_graph_scores.used = false;
-        g_graph_scores.release();
-        /* without it (no memory) the capture records the kernel that needs none */
-        if (!g_graph_scores.ready_ws &&
-            hipMalloc((void **)&g_graph_scores.ready_ws, smq::SCORE_WORKSPACE_BYTES) != hipSuccess) {
-            g_graph_scores.ready_ws = nullptr;
-            (void)hipGetLastError();
-        }
+        GraphScores::drop_all(g_graph_scores.retired);
+        if (!g_graph_scores.ready) g_graph_scores.ready = g_graph_scores.take();
     }
     /* thread-local mode: a call from this thread that may not be captured (a synchronizing copy, an
      * allocation) fails the capture instead of being recorded or run behind the graph's back */
@@ -1476,8 +1537,10 @@ void *smq_capture_end(void) {
     if (mine) {
         std::lock_guard<std::mutex> l(g_graph_scores.mu);
         if (ok && g_graph_scores.used) {
-            g_graph_scores.of_graph[(void *)exec] = g_graph_scores.ready_ws;
-            g_graph_scores.ready_ws = nullptr;
+            g_graph_scores.ready->exec = (void *)exec;
+            g_graph_scores.ready->elsewhere = false;
+            GraphScores::push(g_graph_scores.owned, g_graph_scores.ready);
+            g_graph_scores.ready = nullptr;
         }
         g_graph_scores.used = g_graph_scores.open = false;
     }
@@ -1487,23 +1550,37 @@ void *smq_capture_end(void) {
 smq_status smq_graph_launch(void *graph) {
     if (!ready()) return t_status;
     if (!graph) return set_status(SMQ_ERR_RANGE, "graph is NULL");
-    return hip_ok(hipGraphLaunch((hipGraphExec_t)graph, g.cur), "hipGraphLaunch") ? SMQ_OK : t_status;
+    const hipStream_t s = g.cur;
+    if (s != g.own) {
+        std::lock_guard<std::mutex> l(g_graph_scores.mu);
+        for (GraphScores::Item *i = g_graph_scores.owned; i; i = i->next)
+            if (i->exec == graph) i->elsewhere = true;
+    }
+    return hip_ok(hipGraphLaunch((hipGraphExec_t)graph, s), "hipGraphLaunch") ? SMQ_OK : t_status;
 }
 
 void smq_graph_destroy(void *graph) {
     if (!graph) return;
+    GraphScores::Item *i;
     {
         /* before the handle is free: another thread's capture may get the same one at once */
         std::lock_guard<std::mutex> l(g_graph_scores.mu);
-        auto it = g_graph_scores.of_graph.find(graph);
-        if (it != g_graph_scores.of_graph.end()) {
-            g_graph_scores.retired.push_back(it->second);
-            g_graph_scores.of_graph.erase(it);
-        }
+        i = g_graph_scores.unlink(graph);
     }
     (void)hipGraphExecDestroy((hipGraphExec_t)graph);
     std::lock_guard<std::mutex> l(g_graph_scores.mu);
-    if (!t_capturing) g_graph_scores.release();
+    if (i) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+        if (g.ready && !i->elsewhere && g_graph_scores.spares() < GraphScores::MAX_SPARE &&
+            hipStreamIsCapturing(g.own, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
+            hipEventRecord(i->done, g.own) == hipSuccess) {
+            GraphScores::push(g_graph_scores.spare, i);
+        } else {
+            (void)hipGetLastError();
+            GraphScores::push(g_graph_scores.retired, i);
+        }
+    }
+    if (!t_capturing) GraphScores::drop_all(g_graph_scores.retired);
 }
 
 static bool anchor_shape_ok(const void *a, const void *b, size_t bytes, uint32_t wgs, uint32_t threads) {

@@ -250,7 +250,43 @@ def no_memory():
         smq.smq_graph_destroy(g)
 
 
-CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream, no_memory)]
+def captures_again():
+    """A program that captures its decode step again after each prompt allocates and frees nothing, and a workspace is
+    not handed on while a replay may be using it."""
+    init()
+    att, side = Attention(128), stream()
+    before = fake.fake_allocations(), fake.fake_frees()
+    for _ in range(8):
+        g = capture(att)
+        assert smq.smq_graph_launch(g) == 0
+        assert smq.smq_synchronize() == 0
+        smq.smq_graph_destroy(g)
+    assert (fake.fake_allocations(), fake.fake_frees()) == before
+    for launched_on in (None, side):  # destroyed behind a replay that nobody waited for
+        first = capture(att)
+        smq.smq_set_stream(launched_on)
+        assert smq.smq_graph_launch(first) == 0
+        smq.smq_set_stream(None)
+        smq.smq_graph_destroy(first)
+        second = capture(att)
+        smq.smq_set_stream(stream())
+        assert smq.smq_graph_launch(second) == 0
+        smq.smq_set_stream(None)
+        smq.smq_graph_destroy(second)
+    assert errors() == "", errors()
+    graphs = [capture(att) for _ in range(12)]  # no more kept than a few
+    for g in graphs:
+        smq.smq_graph_destroy(g)
+    assert fake.fake_allocations() - fake.fake_frees() - (before[0] - before[1]) <= 4
+    kept = [capture(att) for _ in range(2)]  # across a shutdown: freed with their graph
+    smq.smq_shutdown()
+    for g in kept:
+        smq.smq_graph_destroy(g)
+    assert errors() == "", errors()
+
+
+CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream, no_memory,
+                     captures_again)]
 
 if __name__ == "__main__":
     load(sys.argv[1])
