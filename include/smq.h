@@ -67,8 +67,9 @@ smq_status smq_set_error(smq_status status, const char *message);
 smq_status smq_init(int device);
 void smq_shutdown(void);
 void *smq_stream(void);                      /* hipStream_t */
-/* NULL restores the library stream. Decode attention at head size 64 keeps its fastest form on every stream as long as
- * a stream of the caller's own is waited for (smq_synchronize, a copy) before another one takes its place. */
+/* NULL restores the library stream. Decode attention at head size 64 has a workspace for the library's stream and two
+ * of the caller's at a time; another one gets it after smq_synchronize, a copy or smq_numeric_check on its stream, and
+ * computes the same without it. */
 smq_status smq_set_stream(void *hip_stream);
 smq_status smq_synchronize(void);
 /* Device name of the selected GPU, e.g. "gfx950". */

@@ -126,16 +126,20 @@ struct GraphScores {
 };
 GraphScores g_graph_scores;
 
-/* Who uses the library's own score workspaces. g.scores, for eager decode attention at head size 64, serves any stream:
- * it passes to another one only when its last use is over (a synchronization of its user through the library) or,
- * from the library's own stream, by an event; no other stream is known to exist still. mu is held while launches that
- * share a workspace are enqueued. */
+/* Score workspaces of eager decode attention at head size 64, for any stream: g.scores for the library's own, and
+ * `other` for the caller's. A stream keeps the one that it has used; another one gets it only when that use is over:
+ * its stream was waited for through the library, or smq_free waited for the device. (An event after each use took 4-8
+ * us, and a stream that is no longer the caller's may not exist any more.) mu is held while launches that share a
+ * workspace are enqueued. */
 struct SharedScores {
+    struct Slot {
+        float *p;
+        hipStream_t user;
+        bool busy;
+        uint64_t uses;
+    };
     std::mutex mu;
-    hipStream_t user = nullptr;
-    bool busy = false;
-    uint64_t uses = 0;
-    hipEvent_t handed = nullptr;
+    Slot other[2] = {};
 };
 SharedScores g_shared;
 
@@ -181,36 +185,42 @@ bool ready() {
     return false;
 }
 
-/* Waits for s, and for the workspace where s used it last. */
-hipError_t finish(hipStream_t s) {
-    uint64_t uses = 0;
+/* Runs wait(), after which the work of s (null: of every stream) is over, and frees the workspaces that only such work
+ * has used. */
+template <typename Wait>
+hipError_t finish(hipStream_t s, Wait wait) {
+    SharedScores &a = g_shared;
+    uint64_t uses[2];
     {
-        std::lock_guard<std::mutex> l(g_shared.mu);
-        if (g_shared.user == s) uses = g_shared.uses;
+        std::lock_guard<std::mutex> l(a.mu);
+        for (int i = 0; i < 2; ++i) uses[i] = a.other[i].uses;
     }
-    const hipError_t e = hipStreamSynchronize(s);
-    std::lock_guard<std::mutex> l(g_shared.mu);
-    if (e == hipSuccess && g_shared.user == s && g_shared.uses == uses) g_shared.busy = false;
+    const hipError_t e = wait();
+    std::lock_guard<std::mutex> l(a.mu);
+    for (int i = 0; i < 2; ++i)
+        if (e == hipSuccess && (!s || a.other[i].user == s) && a.other[i].uses == uses[i]) a.other[i].busy = false;
     return e;
 }
+hipError_t finish(hipStream_t s) {
+    return finish(s, [s] { return hipStreamSynchronize(s); });
+}
 
-/* g.scores for s's next launches, or null. g_shared.mu is held. */
+/* The workspace of s's next launches, or null. g_shared.mu is held. */
 float *take_scores(hipStream_t s) {
-    if (g_shared.busy && g_shared.user != s) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
-        if (g_shared.user != g.own || hipStreamIsCapturing(g.own, &capture) != hipSuccess ||
-            capture != hipStreamCaptureStatusNone)
-            return nullptr;
-        if (hipEventRecord(g_shared.handed, g.own) != hipSuccess ||
-            hipStreamWaitEvent(s, g_shared.handed, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
+    if (s == g.own) return g.scores;
+    SharedScores::Slot *free_slot = nullptr;
+    for (SharedScores::Slot &o : g_shared.other) {
+        if (o.p && o.busy && o.user == s) {
+            ++o.uses;
+            return o.p;
         }
+        if (o.p && !o.busy) free_slot = &o;
     }
-    g_shared.user = s;
-    g_shared.busy = true;
-    ++g_shared.uses;
-    return g.scores;
+    if (!free_slot) return nullptr;
+    free_slot->user = s;
+    free_slot->busy = true;
+    ++free_slot->uses;
+    return free_slot->p;
 }
 
 /* The byte range [p, p + bytes) must lie inside one device allocation. */
@@ -392,7 +402,13 @@ smq_status smq_init(int device) {
         g.tiles_ws = nullptr;
         (void)hipGetLastError();
     }
-    if (!hip_ok(hipEventCreateWithFlags(&g_shared.handed, hipEventDisableTiming), "hipEventCreate")) return t_status;
+    for (SharedScores::Slot &o : g_shared.other) {
+        o = SharedScores::Slot();
+        if (hipMalloc((void **)&o.p, smq::SCORE_WORKSPACE_BYTES) != hipSuccess) {
+            o.p = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     if (!hip_ok(hipEventCreate(&g.t0), "hipEventCreate") || !hip_ok(hipEventCreate(&g.t1), "hipEventCreate"))
         return t_status;
     /* the allocation-free argmax's static partials: their device address, once, with the device current */
@@ -422,9 +438,10 @@ void smq_shutdown(void) {
     (void)hipStreamSynchronize(g.cur);
     (void)hipEventDestroy(g.t0);
     (void)hipEventDestroy(g.t1);
-    (void)hipEventDestroy(g_shared.handed);
-    g_shared.user = nullptr;
-    g_shared.busy = false;
+    for (SharedScores::Slot &o : g_shared.other) {
+        (void)hipFree(o.p);
+        o = SharedScores::Slot();
+    }
     (void)hipFree(g.flag);
     (void)hipFree(g.argmax_parts);
     (void)hipFree(g.scores);
@@ -1459,7 +1476,7 @@ void smq_free(void *p) {
         std::lock_guard<std::mutex> lock(g_alloc_mu);
         g_allocs.erase((uintptr_t)p);
     }
-    (void)hipFree(p);
+    (void)finish(nullptr, [p] { return hipFree(p); }); /* waits for the device */
 }
 
 smq_status smq_memcpy_htod(void *dst, const void *src, size_t bytes) {

@@ -206,14 +206,18 @@ def scores_by_stream():
             assert att() == 0
             assert two_launches() == expected and errors() == "", fake.fake_log().decode() + errors()
 
-        call(side, not split)  # from the library's stream to another: in order by an event
-        call(None, split)  # the other stream's use may be running: the launch that needs no workspace
-        call(third, False)
+        fourth = stream()
+        for s in (side, None, third, side, None, third):  # a workspace for each of three streams, without a wait
+            call(s, not split or s is None)
+        call(fourth, False)  # the launch that needs none
         call(side, not split)
         assert smq.smq_synchronize() == 0
-        for s in (third, side, None):  # after a synchronization of its user every stream may have it
+        call(fourth, not split)  # the other's use is over
+        call(side, False)
+        smq.smq_free(smq.smq_malloc(64))  # waits for the device
+        for s in (side, fourth, None):
             call(s, not split or s is None)
-            assert smq.smq_synchronize() == 0
+        call(third, False)
 
         for s in (side, own):  # a capture that the program opened itself
             smq.smq_set_stream(s)
