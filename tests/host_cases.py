@@ -66,14 +66,14 @@ def on_thread(f):
 
 
 class Attention:
-    """One token's attention (ntok: up to 256) with buffers of its own."""
+    """One token's attention (ntok: up to 512) with buffers of its own."""
 
     def __init__(self, hd, heads=4, kv=2, context=2048, window=0):
         self.shape = Shape(heads, kv, hd, hd // 2, window, context)
         self.heads, self.hd, self.kvd, self.context = heads, hd, kv * hd, context
         self.cache = [smq.smq_malloc(context * self.kvd * 4) for _ in range(2)]
         self.pos = smq.smq_malloc(4)
-        self.rows = [smq.smq_malloc(256 * heads * hd * 4) for _ in range(2)]
+        self.rows = [smq.smq_malloc(512 * heads * hd * 4) for _ in range(2)]
 
     def __call__(self, pos=1000, ntok=1, pos_dev=False):
         q, att = self.rows
@@ -289,8 +289,97 @@ def captures_again():
     assert errors() == "", errors()
 
 
+def tile_routes():
+    """Every shape of the GPU test of the attention tiles reaches them, and none in a capture or on another stream."""
+    sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+    from test_gpu_attend_tiles import CASES as SHAPES
+    init()
+    side = stream()
+    for heads, kv, hd, window, context, ntok, pos0 in SHAPES:
+        att = Attention(hd, heads, kv, context, window)
+        for s in (None, side):
+            smq.smq_set_stream(s)
+            fake.fake_clear()
+            assert att(pos0, ntok) == 0, smq.smq_last_error()
+            names = kernels()
+            tiles = [any(k in n for n in names) for k in ("k_ap_scores", "k_ap_softmax", "k_ap_values")]
+            assert tiles == [s is None] * 3, (heads, kv, hd, window, context, ntok, pos0, names)
+        smq.smq_set_stream(None)
+        fake.fake_clear()
+        assert smq.smq_graph_launch(capture(lambda: att(pos0, ntok))) == 0
+        assert not any("k_ap" in n for n in kernels())
+
+
+def attention_routes():
+    """Both sides of the lines between the prefill kernels and between the decode kernels."""
+    init()
+    prefill = [  # heads, kv_heads, hd, window, context, ntok, pos0, kernel
+        (14, 2, 64, 0, 1024, 512, 0, "k_ap_"), (14, 2, 64, 0, 1024, 2, 256, "k_attend_group"),
+        (14, 2, 64, 0, 1024, 2, 1000, "k_ap_"), (9, 3, 64, 512, 964, 17, 564, "k_attend_group"),
+        (9, 3, 64, 0, 644, 16, 572, "k_attend_group"), (32, 8, 64, 512, 853, 61, 718, "k_attend_group"),
+        (32, 8, 64, 0, 363, 89, 202, "k_ap_"), (14, 2, 64, 128, 2002, 22, 331, "k_attend_rows"),
+        (9, 3, 64, 128, 5078, 40, 3276, "k_attend_rows"), (14, 2, 64, 0, 2002, 16, 1000, "k_attend_rows"),
+        (14, 2, 64, 0, 4000, 16, 3800, "k_ap_"), (12, 2, 128, 0, 3100, 8, 3000, "k_ap_"),
+        (12, 2, 128, 0, 600, 4, 500, "k_attendE"), (16, 2, 36, 0, 3100, 64, 3000, "k_attendE"),
+    ]
+    decode = [  # heads, kv_heads, hd, window, context, pos, kernel
+        (14, 2, 64, 0, 2048, 5, "k_attend_values"), (12, 2, 128, 0, 2048, 150, "k_attendE"),
+        (12, 2, 128, 0, 2048, 151, "k_attend_values"), (12, 2, 128, 100, 2048, 1000, "k_attendE"),
+        (9, 3, 32, 0, 2048, 246, "k_attendE"), (9, 3, 32, 0, 2048, 247, "k_attend_values"),
+        (17, 1, 128, 0, 2048, 1000, "k_attendE"), (17, 1, 64, 0, 2048, 1000, "k_attend_rows"),
+        (9, 3, 48, 0, 2048, 1000, "k_attendE"),
+    ]
+    for heads, kv, hd, window, context, *rest in prefill + [(*d[:5], 1, *d[5:]) for d in decode]:
+        ntok, pos, want = rest
+        att = Attention(hd, heads, kv, context, window)
+        fake.fake_clear()
+        assert att(pos, ntok) == 0, smq.smq_last_error()
+        assert want in kernels()[-1], (heads, kv, hd, window, context, rest, kernels())
+
+
+def matmul_routes():
+    """Both sides of the lines between the kernels of 2-16 tokens (256 CUs)."""
+    sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+    from smq_pkg import smq as package
+    QMat, Item = package._QMat, package._MatItem
+    init()
+    w, x, y = (smq.smq_malloc(1 << 30) for _ in range(3))
+    four, wide = "k_gemm_xmILb%dELb0ELi4E", "k_gemm_xmILb%dELb0ELi1E"
+    dot8, dot16, few = "k_gemm_exactILb%dELb0ELi8E", "k_gemm_exactILb%dELb0ELi16E", "k_gemv_fewILb%d"
+    table = [  # rows, cols, ntok, Q8, Q5
+        (4096, 896, 12, dot8, dot8), (4128, 896, 12, four, four), (4864, 4864, 11, four, four),
+        (4864, 384, 16, dot8, dot8), (4864, 448, 16, four, four), (5120, 384, 16, four, four),
+        (14304, 576, 16, four, four), (14336, 576, 16, wide, wide), (24576, 576, 9, wide, wide), (24576, 896, 9, four, four),
+        (65536, 896, 16, wide, wide), (65504, 896, 16, four, four), (16384, 896, 8, dot8, dot8),
+        (2048, 448, 4, few, few), (2688, 448, 4, dot8, dot8), (16384, 1536, 4, few, dot8), (16400, 1536, 4, dot8, dot8),
+        (12288, 1536, 3, few, few), (4096, 896, 2, few, few), (4128, 896, 2, few, dot8), (1024, 1536, 12, few, few),
+        (1024, 896, 16, dot8, dot8), (1024, 1984, 16, few, few),
+    ]
+    for rows, cols, ntok, *wants in table:
+        for q5, want in enumerate(wants):
+            nb = (cols + 31) // 32
+            m = QMat(w, rows, cols, nb, package.DTYPE_Q5 if q5 else package.DTYPE_Q8, nb * (22 if q5 else 36))
+            item = Item(ctypes.pointer(m), None, y, 0)
+            fake.fake_clear()
+            assert smq.smq_matmul(ctypes.byref(item), 1, x, x, ntok) == 0, smq.smq_last_error()
+            assert want % q5 in kernels()[0], (rows, cols, ntok, q5, kernels())
+
+
+def conversion_limits():
+    """Q5 conversion: both sides of the line between one and two rounds, and the most blocks (addresses only)."""
+    init()
+    x, out = smq.smq_malloc(18 << 30), smq.smq_malloc(95 << 30)
+    for rows, kernel, grid in ((1, "Lj1E", 1), (28000, "Lj1E", 2334), (28001, "Lj2E", 1167),
+                               (2**32 - 1, "Lj2E", (2**32 - 1 + 23) // 24)):
+        fake.fake_clear()
+        assert smq.smq_quantize_q5_rows(x, rows, 1, out) == 0, smq.smq_last_error()
+        assert kernel in kernels()[0] and int(log()[0][2]) == grid, log()
+    fake.fake_clear()
+    assert smq.smq_quantize_q5_rows(x, 2**31, 65, out) != 0 and not log()  # past both allocations
+
+
 CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream, no_memory,
-                     captures_again)]
+                     captures_again, tile_routes, attention_routes, matmul_routes, conversion_limits)]
 
 if __name__ == "__main__":
     load(sys.argv[1])
