@@ -85,3 +85,46 @@ def test_attend_tiles_later_rows_do_not_reach_earlier_tokens(orc):
     got = att.download(np.float32).reshape(ntok, qd)
     assert_same_f32(got[:5], want, "tokens before the non-finite row")
     assert not np.isfinite(got[5:]).any()
+
+
+@pytest.mark.parametrize("scale", ["spread", "tiny"])
+@pytest.mark.parametrize("heads,kv_heads,hd,context,ntok,pos0", [(14, 2, 64, 1100, 20, 1010), (12, 2, 128, 700, 11, 645),
+                                                                 (8, 4, 16, 200, 101, 70)])
+def test_attend_tiles_small_values(orc, scale, heads, kv_heads, hd, context, ntok, pos0):
+    """Weights that are subnormal or zero (a wide spread of scores); scores, values and products that are subnormal."""
+    say("attend tiles", scale, heads, hd)
+    qd, kd = heads * hd, kv_heads * hd
+    qs, ks, vs = (30.0, 1.0, 1.0) if scale == "spread" else (1e-20, 1e-20, 3e-39)
+    q = synth.normal(47, ntok * qd, qs).reshape(ntok, qd)
+    keys = synth.normal(48, context * kd, ks).reshape(context, kd)
+    values = synth.normal(49, context * kd, vs).reshape(context, kd)
+    att = smq.DeviceBuffer(ntok * qd * 4)
+    smq.attention(dev(q), dev(keys), dev(values), att, ntok, smq.attn_shape(heads, kv_heads, hd, hd // 2, 0, context), pos0)
+    smq.synchronize()
+    want = attend_expect(orc, q, keys, values, heads, kv_heads, hd, 0, pos0, ntok)
+    assert np.isfinite(want).all() and want.any()
+    assert_same_f32(att.download(np.float32).reshape(ntok, qd), want, scale)
+
+
+@pytest.mark.parametrize("what", ["inf value", "inf - inf", "nan value", "nan key", "inf key", "-inf key"])
+@pytest.mark.parametrize("heads,kv_heads,hd,context,ntok,pos0", [(14, 2, 64, 1400, 20, 1010), (12, 2, 128, 1400, 11, 645),
+                                                                 (14, 2, 64, 1400, 1, 1300), (6, 2, 96, 1400, 1, 1300)])
+def test_attend_non_finite(orc, what, heads, kv_heads, hd, context, ntok, pos0):
+    """Non-finite keys and values among the positions that the rows see, in the tiles and in the long value path."""
+    say("attend", what, heads, hd, ntok)
+    qd, kd = heads * hd, kv_heads * hd
+    q = synth.normal(57, ntok * qd).reshape(ntok, qd)
+    keys = synth.normal(58, context * kd).reshape(context, kd)
+    values = synth.normal(59, context * kd).reshape(context, kd)
+    at = pos0 - 20
+    if what.endswith("key"):
+        keys[at, kd - hd + 5] = {"nan key": np.nan, "inf key": np.inf, "-inf key": -np.inf}[what]
+    else:
+        values[at, 3] = np.nan if what == "nan value" else np.inf
+        if what == "inf - inf":
+            values[at + 9, 3] = -np.inf
+    att = smq.DeviceBuffer(ntok * qd * 4)
+    smq.attention(dev(q), dev(keys), dev(values), att, ntok, smq.attn_shape(heads, kv_heads, hd, hd // 2, 0, context), pos0)
+    smq.synchronize()
+    want = attend_expect(orc, q, keys, values, heads, kv_heads, hd, 0, pos0, ntok)
+    assert_same_f32(att.download(np.float32).reshape(ntok, qd), want, what)
