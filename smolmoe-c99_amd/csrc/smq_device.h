@@ -484,11 +484,10 @@ __constant__ uint64_t EXP2_TABLE[32] = {
 /* e^x in binary64, rounded once (vecmath.c:61-76): k = round(32x/ln2) from the
  * low bits of z + 1.5*2^52, remainder r, degree-4 Taylor polynomial of
  * e^(r ln2/32) with separate multiplies and adds, times 2^(k/32). */
-__device__ __forceinline__ float exp_det_tab(float x, const uint64_t *tab) {
+__device__ __forceinline__ float exp_det_value(float x, const uint64_t *tab) { /* x: not a NaN */
     const double inv_ln2_n = 0x1.71547652b82fep+5, shift = 0x1.8p+52;
     const double ea = 0x1.62e42fefa39efp-1 / 32;
     const double c1 = ea, c2 = ea * ea / 2, c3 = ea * ea * ea / 6, c4 = ea * ea * ea * ea / 24;
-    if (x != x) return x;
     x = x > 89.0f ? 89.0f : (x < -104.0f ? -104.0f : x);
     const double z = inv_ln2_n * (double)x;
     double kd = z + shift;
@@ -502,28 +501,17 @@ __device__ __forceinline__ float exp_det_tab(float x, const uint64_t *tab) {
     const double scale = __longlong_as_double((long long)(tab[ki & 31u] + (ki << 47)));
     return (float)(p * scale);
 }
-
-__device__ __forceinline__ float exp_det(float x) { return exp_det_tab(x, EXP2_TABLE); }
-
-/* exp_det_tab without a branch: several of a thread's run side by side. */
+__device__ __forceinline__ float exp_det_tab(float x, const uint64_t *tab) {
+    if (x != x) return x;
+    return exp_det_value(x, tab);
+}
+/* The same without a branch: several of a thread's run side by side. */
 __device__ __forceinline__ float exp_det_flat(float x, const uint64_t *tab) {
-    const double inv_ln2_n = 0x1.71547652b82fep+5, shift = 0x1.8p+52;
-    const double ea = 0x1.62e42fefa39efp-1 / 32;
-    const double c1 = ea, c2 = ea * ea / 2, c3 = ea * ea * ea / 6, c4 = ea * ea * ea * ea / 24;
-    const float xc = x > 89.0f ? 89.0f : (x < -104.0f ? -104.0f : x);
-    const double z = inv_ln2_n * (double)xc;
-    double kd = z + shift;
-    const uint64_t ki = (uint64_t)__double_as_longlong(kd);
-    kd = kd - shift;
-    const double r = z - kd;
-    double p = c4 * r + c3;
-    p = p * r + c2;
-    p = p * r + c1;
-    p = p * r + 1.0;
-    const double scale = __longlong_as_double((long long)(tab[ki & 31u] + (ki << 47)));
-    const float e = (float)(p * scale);
+    const float e = exp_det_value(x, tab);
     return x != x ? x : e;
 }
+
+__device__ __forceinline__ float exp_det(float x) { return exp_det_tab(x, EXP2_TABLE); }
 
 /* DPP move of v from another lane of its row of 16 (ctrl: a dpp_ctrl code). */
 template <int CTRL>
