@@ -15,9 +15,10 @@
  * 128 adds 281 ns; 128 v_mul and 128 v_add 231 ns, but 342 ns when the common
  * operand comes by DPP, and scalar loads of it did not keep up.
  * 256 tokens at positions 3328-3583, 12 heads of 128 over 2 KV heads: 4220 us
- * with a workgroup per token, head and 32 columns -> 171 us (scores 72,
- * softmax 30, values 88; the products and adds alone need about 46 + 46 at
- * four waves per SIMD, and this many rows fill less than two). */
+ * with a workgroup per token, head and 32 columns -> 171 us (traced one by
+ * one, with their own start and end, scores 72, softmax 29, values 90; the
+ * products and adds alone need about 46 + 46 at four waves per SIMD, and this
+ * many rows fill less than two). */
 #include "smq_device.h"
 
 namespace smq {

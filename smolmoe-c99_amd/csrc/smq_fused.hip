@@ -202,7 +202,7 @@ k_gemv_fused(FusedArgs a, uint32_t ntiles) {
                 }
             }
             lds_barrier();
-            first_loads(); /* after the serial sum (before it: the same time, 23.6 / 23.4 us below) */
+            first_loads(); /* after the serial sum (before it the FFN above took 23.4 us, not 23.6: the spread of the runs) */
             const float inv = s_inv;
             if (tid == 0 && s_bad && a.flag) *a.flag = 1;
             /* (x*inv)*w and its Q8 blocks; uniform: a block's 32 lanes are all below np or past it */

@@ -155,7 +155,7 @@ __global__ __launch_bounds__(WG) void k_gemv(MatArgs a) {
  * 2-16 tokens against few or long rows, FEW_NT tokens per pass: k_gemv's tasks, each with its block's words of every
  * token of the pass. The products spread over all threads and only the adds stay serial, a thread per (token, row,
  * lane), where a thread per output (k_gemm_exact) leaves few rows a serial chain of products and a chunk of 16 blocks
- * in flight: 896x4864 at 4 tokens 22.5 -> 6.3 us, Q5 1536x8960 at 4 39.3 -> 10.5, 2048x2048 at 8 11.9 -> 6.2. A task
+ * in flight: 896x4864 at 4 tokens 22.5 -> 5.7 us, Q5 1536x8960 at 4 39.3 -> 10.5, 2048x2048 at 8 11.9 -> 6.2. A task
  * decodes its weights once for all passes; the next pass's or chunk's loads are in flight during the products and
  * adds. What bounds it with many rows is the LDS traffic of the products, a write and a read each: few_wanted.
  * ---------------------------------------------------------------------- */
@@ -1627,15 +1627,15 @@ __global__ __launch_bounds__(ATT_WG) void k_attend(const float *q, const float *
  * the two serial sums.
  *  0. every load is issued first: the K rows of up to AR_KR positions
  *     (coalesced: 16 threads per row, AR_KU float4 per thread held in
- *     registers), the first AR_VP value rows of this workgroup's 32
+ *     registers), up to AR_VP positions the value rows of this workgroup's 32
  *     coordinates, q and the exp table;
  *  1. scores: the rows pass through LDS AR_KT at a time; one thread per
  *     position forms the 8-lane dot_f32 of kernels.c:1119-1127 (lane tree,
  *     times 1/sqrt(hd));
  *  2. maximum (order-free) and exp_det(s - max) in parallel;
  *  3. the total in position order by one lane, inv = 1/total;
- *  4. the products (s_p*inv)*v_p[j] of AR_VP rows at a time to LDS, then lane
- *     j adds its column in position order while the next rows load.
+ *  4. the products (s_p*inv)*v_p[j] to LDS, then lane j adds its column in
+ *     position order; past AR_VP positions chunk by chunk (att_long).
  * ROPE (one token, decode): q and this position's k arrive unrotated, as the
  * QKV matmul left them; the workgroup rotates q and this position's k row
  * into LDS (model.c:442-450, 511-526), and the first workgroup of each KV
@@ -2074,7 +2074,8 @@ __global__ __launch_bounds__(AS_WG) void k_attend_scores(const float *q, float *
     }
 }
 
-/* The scores of other head sizes (multiples of 8): the same pairs of threads, the head's size at run time. */
+/* The scores of other head sizes (the kernel takes multiples of 8, its callers 32: k_attend_values): the same pairs of
+ * threads, the head's size at run time. */
 __global__ __launch_bounds__(AS_WG) void k_attend_scores_hd(const float *q, const float *kcache, AttnShape sh,
                                                             uint32_t pos0, const int32_t *pos_dev, int *flag,
                                                             float *scores) {
