@@ -608,8 +608,10 @@ def capture(fn):
     _check(lib.smq_capture_begin())
     try:
         fn()
-    finally:
-        handle = lib.smq_capture_end()
+    except BaseException:
+        lib.smq_graph_destroy(lib.smq_capture_end())  # what was recorded, and its workspace, go with the exception
+        raise
+    handle = lib.smq_capture_end()
     if not handle:
         _check()
     return Graph(handle)

@@ -378,8 +378,30 @@ def conversion_limits():
     assert smq.smq_quantize_q5_rows(x, 2**31, 65, out) != 0 and not log()  # past both allocations
 
 
+def capture_with_an_exception():
+    """The binding's capture of a function that raises leaves neither a graph nor its workspace behind."""
+    sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+    from smq_pkg import smq as package
+    init()
+    package.load()
+    att, before = Attention(128), fake.fake_allocations()
+
+    def broken():
+        assert att() == 0
+        raise KeyError("in the middle")
+
+    for _ in range(5):
+        try:
+            package.capture(broken)
+        except KeyError:
+            continue
+        raise AssertionError("no exception")
+    assert fake.fake_allocations() == before and errors() == "", errors()
+    package.capture(lambda: att()).destroy()
+
+
 CASES = [f for f in (nested_capture, failed_captures, destroyed_handle, stream_read_once, scores_by_stream, no_memory,
-                     captures_again, tile_routes, attention_routes, matmul_routes, conversion_limits)]
+                     captures_again, capture_with_an_exception, tile_routes, attention_routes, matmul_routes, conversion_limits)]
 
 if __name__ == "__main__":
     load(sys.argv[1])
