@@ -11,13 +11,13 @@
  * (denormals kept; an underflow to -0 instead of +0 changes no sum that holds
  * a nonzero term), and the VALU does the adds. A tile is 16 rows that share a
  * KV head, so each K and V row read serves 16 rows, and neither operand needs
- * a broadcast. Measured per SIMD with four waves: 8 such products and their
- * 128 adds 281 ns; 128 v_mul and 128 v_add 231 ns, but 342 ns when the common
+ * a broadcast. Measured per wave with four on a SIMD: 8 such products and their
+ * 128 adds 247 ns; 128 v_mul and 128 v_add 231 ns, but 302 ns when the common
  * operand comes by DPP, and scalar loads of it did not keep up.
  * 256 tokens at positions 3328-3583, 12 heads of 128 over 2 KV heads: 4220 us
  * with a workgroup per token, head and 32 columns -> 171 us (traced one by
  * one, with their own start and end, scores 72, softmax 29, values 90; the
- * products and adds alone need about 46 + 46 at four waves per SIMD, and this
+ * products and adds alone need about 40 + 40 at four waves per SIMD, and this
  * many rows fill less than two). */
 #include "smq_device.h"
 

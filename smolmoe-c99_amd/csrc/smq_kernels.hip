@@ -157,7 +157,8 @@ __global__ __launch_bounds__(WG) void k_gemv(MatArgs a) {
  * lane), where a thread per output (k_gemm_exact) leaves few rows a serial chain of products and a chunk of 16 blocks
  * in flight: 896x4864 at 4 tokens 22.5 -> 5.7 us, Q5 1536x8960 at 4 39.3 -> 10.5, 2048x2048 at 8 11.9 -> 6.2. A task
  * decodes its weights once for all passes; the next pass's or chunk's loads are in flight during the products and
- * adds. What bounds it with many rows is the LDS traffic of the products, a write and a read each: few_wanted.
+ * adds. Neither the VALU nor LDS is full (16384x896 at 4 tokens: 30 and 18 % busy): what is left are the barriers
+ * between the products and the adds, which the tile kernels pay once per chunk for more outputs: few_wanted.
  * ---------------------------------------------------------------------- */
 constexpr int FEW_NT = 4; /* tokens per pass */
 template <bool Q5, bool FAST, int RT, int NG>
