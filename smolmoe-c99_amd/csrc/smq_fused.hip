@@ -132,12 +132,11 @@ k_gemv_fused(FusedArgs a, uint32_t ntiles) {
     auto load_task = [&](const Row &R, uint32_t b) __attribute__((always_inline)) { load_words(R, b, wr); };
     Row cur, nxt;
     setup(t0, cur);
+    if constexpr (ONE) setup(t0 + 1 < t1 ? t0 + 1 : t0, nxt);
     auto first_loads = [&]() __attribute__((always_inline)) {
         load_words(cur, ti * TB, wr);
-        if constexpr (ONE) {
-            setup(t0 + 1 < t1 ? t0 + 1 : t0, nxt);
-            load_words(nxt, ti * TB, wn);
-        }
+        if constexpr (ONE)
+            if (t0 + 1 < t1) load_words(nxt, ti * TB, wn); /* uniform */
     };
 
     /* prologue: the activation into LDS. Rows of up to FU_SHORT elements per thread load x (and
